@@ -182,11 +182,20 @@ int pad_decode_workspace_bytes(const pad_decode_dims* dims, int num_splits,
 /* int32 arrival counters a launch with these arguments needs (0 when the
  * plan is single-pass; otherwise U = batch * num_kv_heads, or U * (1 +
  * num_splits) when U * num_splits > 48, so that a sequence may get more
- * than 48 split items and merge them in two levels).  Pure host
+ * than 48 split items and merge them in two levels; at least what the range
+ * kernel counts with, where a launch may take it).  Pure host
  * function.  No counterpart in the reference, whose two kernel launches
  * needed no arrival counting. */
 int pad_decode_counters_needed(const pad_decode_dims* dims, int num_splits,
                                int num_cus, int64_t* count);
+
+/* The least workspace and counters that a launch with these arguments (csr =
+ * 1 for a CSR index) accepts: the per-unit kernel's, at most what
+ * pad_decode_workspace_bytes() / pad_decode_counters_needed() return.  A
+ * launch with less than those runs that kernel.  Pure host function. */
+int pad_decode_least_scratch(const pad_decode_dims* dims, int num_splits,
+                             int num_cus, int csr, size_t* bytes,
+                             int64_t* count);
 
 /* pad_decode_launch() without workspace or counters arguments: it allocates
  * nothing (no hipMalloc/hipFree, no allocating library call), for callers

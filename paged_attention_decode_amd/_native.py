@@ -124,6 +124,11 @@ SIGNATURES = {
         [ctypes.POINTER(PadDims), ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int64)],
         ctypes.c_int,
     ),
+    "pad_decode_least_scratch": (
+        [ctypes.POINTER(PadDims), ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_size_t),
+         ctypes.POINTER(ctypes.c_int64)],
+        ctypes.c_int,
+    ),
     "pad_decode_counters_init": ([_VP, ctypes.c_int64, _VP], ctypes.c_int),
     "pad_decode_launch": (
         [_VP, _VP, _VP, _VP, _VP, _VP, _VP, ctypes.c_size_t, _VP, ctypes.c_int64, ctypes.POINTER(PadDims),

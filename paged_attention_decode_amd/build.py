@@ -5,7 +5,7 @@ below):
 
 * ``libpa_decode.so`` - the C-ABI library (``include/pa_decode.h``): gfx950
   kernels plus ``extern "C"`` entry points, compiled by ``hipcc`` from
-  ``csrc/pa_decode.hip``.
+  ``csrc/pa_decode.hip`` and ``csrc/pa_range.hip``.
 * ``_pa_decode_ext<EXT_SUFFIX>`` - the thin PyTorch binding
   (``csrc/pa_torch.cpp``), host-only C++ compiled by ``g++`` against
   PyTorch's headers and linked to ``libpa_decode.so`` through an
@@ -22,7 +22,7 @@ host C++ linked to ``libpa_decode.so`` and the HIP runtime), a compiled
 caller of the C ABI that ``tests/test_capi_consumer.py`` runs.
 
 Usage: ``python -m paged_attention_decode_amd.build`` (or ``build()`` from
-``__graft_entry__``).  Every call recompiles; the three hipcc builds run in
+``__graft_entry__``).  Every call recompiles; the hipcc builds run in
 parallel.
 """
 
@@ -41,6 +41,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(REPO_DIR, "include")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = "gfx950"
+CAPI_SOURCES = ("pa_decode", "pa_range")  # csrc/*.hip of libpa_decode.so
 
 CAPI_LIB = os.path.join(PKG_DIR, "libpa_decode.so")
 PROBE_LIB = os.path.join(PKG_DIR, "libpa_probe.so")
@@ -78,7 +79,16 @@ def _run(cmd: list[str]) -> None:
 def build_capi() -> str:
     hipcc = os.path.join(ROCM, "bin", "hipcc")
     tmp = CAPI_LIB + ".tmp"
-    _run([hipcc, *HIP_FLAGS, f"-I{INCLUDE}", os.path.join(CSRC, "pa_decode.hip"), "-o", tmp])
+    flags = [f for f in HIP_FLAGS if f != "-shared"]
+    objects = [os.path.join(PKG_DIR, name + ".o") for name in CAPI_SOURCES]
+    with ThreadPoolExecutor(max_workers=len(objects)) as pool:
+        jobs = [pool.submit(_run, [hipcc, *flags, f"-I{INCLUDE}", "-c", os.path.join(CSRC, name + ".hip"), "-o", obj])
+                for name, obj in zip(CAPI_SOURCES, objects)]
+        for job in jobs:
+            job.result()
+    _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", tmp])
+    for obj in objects:
+        os.remove(obj)
     os.replace(tmp, CAPI_LIB)
     return CAPI_LIB
 

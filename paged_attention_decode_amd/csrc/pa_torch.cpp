@@ -21,6 +21,7 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstdint>
 #include <cstring>
@@ -70,8 +71,11 @@ bool stream_capturing(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
+// `least_ws` / `least_counters`: what the launch can do with (the per-unit
+// kernel's scratch); during capture a stream that holds that much is used as
+// it is.
 StreamScratch& stream_scratch(const torch::Tensor& like, hipStream_t stream, size_t ws_bytes,
-                              int64_t num_counters) {
+                              int64_t num_counters, size_t least_ws, int64_t least_counters) {
   static std::mutex mu;
   static std::map<std::pair<int, uintptr_t>, StreamScratch> cache;
   std::lock_guard<std::mutex> lock(mu);
@@ -79,10 +83,13 @@ StreamScratch& stream_scratch(const torch::Tensor& like, hipStream_t stream, siz
   const bool grow_ws = !sc.workspace.defined() || static_cast<size_t>(sc.workspace.numel()) < ws_bytes;
   const bool grow_cnt = !sc.counters.defined() || sc.counters.numel() < num_counters;
   if ((grow_ws || grow_cnt) && stream_capturing(stream)) {
-    TORCH_CHECK(false,
+    const size_t have_ws = sc.workspace.defined() ? static_cast<size_t>(sc.workspace.numel()) : 0;
+    const int64_t have_counters = sc.counters.defined() ? sc.counters.numel() : 0;
+    TORCH_CHECK(have_ws >= least_ws && have_counters >= least_counters,
                 "pa_decode: this call needs more split scratch than the capturing stream holds, and scratch "
                 "cannot grow during HIP graph capture (a captured graph keeps the addresses it was captured "
                 "with). Run one eager call with the largest shape on the capture stream before capturing.");
+    return sc;
   }
   if (grow_ws) {
     const size_t old = sc.workspace.defined() ? static_cast<size_t>(sc.workspace.numel()) : 0;
@@ -99,6 +106,33 @@ StreamScratch& stream_scratch(const torch::Tensor& like, hipStream_t stream, siz
     sc.counters = torch::zeros({grown}, like.options().dtype(at::kInt));
   }
   return sc;
+}
+
+// The stream's scratch as one launch of plan (dims d) gets it: as much of it as
+// the plan asks for, or less during capture (see stream_scratch).
+struct LaunchScratch {
+  void* workspace = nullptr;
+  size_t workspace_bytes = 0;
+  int32_t* counters = nullptr;
+  int64_t num_counters = 0;
+};
+
+LaunchScratch launch_scratch(const torch::Tensor& q, hipStream_t stream, const pad_decode_dims& d, int num_splits,
+                             int cus, bool csr, const pad_decode_plan_t& plan) {
+  LaunchScratch s;
+  if (plan.single_pass) return s;
+  size_t least_ws = 0;
+  int64_t least_counters = 0;
+  const int st = pad_decode_least_scratch(&d, num_splits, cus, csr ? 1 : 0, &least_ws, &least_counters);
+  TORCH_CHECK(st == PAD_OK, "pa_decode: ", pad_status_string(st));
+  StreamScratch& sc = stream_scratch(q, stream, plan.workspace_bytes, plan.counters, least_ws, least_counters);
+  if (sc.workspace.defined() && sc.counters.defined()) {
+    s.workspace = sc.workspace.data_ptr();
+    s.workspace_bytes = std::min(plan.workspace_bytes, static_cast<size_t>(sc.workspace.numel()));
+    s.counters = sc.counters.data_ptr<int32_t>();
+    s.num_counters = std::min<int64_t>(plan.counters, sc.counters.numel());
+  }
+  return s;
 }
 
 void fill_dims(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& v,
@@ -222,13 +256,11 @@ torch::Tensor launch_call(const torch::Tensor& q, const torch::Tensor& k_cache, 
   c.indptr = ix.indptr;
   c.last_page_len = ix.last_page_len;
   c.out = out.data_ptr();
-  if (!plan.single_pass) {
-    StreamScratch& sc = stream_scratch(q, stream, plan.workspace_bytes, plan.counters);
-    c.workspace = sc.workspace.data_ptr();
-    c.workspace_bytes = plan.workspace_bytes;
-    c.counters = sc.counters.data_ptr<int32_t>();
-    c.num_counters = plan.counters;
-  }
+  const LaunchScratch scratch = launch_scratch(q, stream, d, static_cast<int>(num_splits), cus, csr, plan);
+  c.workspace = scratch.workspace;
+  c.workspace_bytes = scratch.workspace_bytes;
+  c.counters = scratch.counters;
+  c.num_counters = scratch.num_counters;
   if (worklist.defined()) {
     c.worklist = worklist.data_ptr();
     c.worklist_bytes = static_cast<size_t>(worklist.numel());
@@ -265,16 +297,11 @@ torch::Tensor forward(torch::Tensor q, torch::Tensor k_cache, torch::Tensor v_ca
   int st = pad_decode_plan(&d, static_cast<int>(num_splits), cus, &plan);
   TORCH_CHECK(st == PAD_OK, "pa_decode: ", pad_status_string(st));
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.get_device()).stream();
-  void* ws_ptr = nullptr;
-  int32_t* counters = nullptr;
-  if (!plan.single_pass) {
-    StreamScratch& sc = stream_scratch(q, stream, plan.workspace_bytes, plan.counters);
-    ws_ptr = sc.workspace.data_ptr();
-    counters = sc.counters.data_ptr<int32_t>();
-  }
+  const LaunchScratch scratch = launch_scratch(q, stream, d, static_cast<int>(num_splits), cus, false, plan);
   st = pad_decode_launch_ex(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                             block_table.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(), out.data_ptr(),
-                            ws_ptr, plan.workspace_bytes, counters, plan.counters, &d, static_cast<float>(scale),
+                            scratch.workspace, scratch.workspace_bytes, scratch.counters, scratch.num_counters, &d,
+                            static_cast<float>(scale),
                             static_cast<int>(num_splits), static_cast<int>(engine), nullptr, stream);
   TORCH_CHECK(st == PAD_OK, "pa_decode: ", pad_status_string(st));
   return out;
@@ -301,16 +328,11 @@ torch::Tensor forward_kv8(torch::Tensor q, torch::Tensor k_cache, torch::Tensor 
   int st = pad_decode_plan(&d, static_cast<int>(num_splits), cus, &plan);
   TORCH_CHECK(st == PAD_OK, "pa_decode: ", pad_status_string(st));
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.get_device()).stream();
-  void* ws_ptr = nullptr;
-  int32_t* counters = nullptr;
-  if (!plan.single_pass) {
-    StreamScratch& sc = stream_scratch(q, stream, plan.workspace_bytes, plan.counters);
-    ws_ptr = sc.workspace.data_ptr();
-    counters = sc.counters.data_ptr<int32_t>();
-  }
+  const LaunchScratch scratch = launch_scratch(q, stream, d, static_cast<int>(num_splits), cus, false, plan);
   st = pad_decode_launch_kv8(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                              block_table.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(), out.data_ptr(),
-                             ws_ptr, plan.workspace_bytes, counters, plan.counters, &d, static_cast<float>(scale),
+                             scratch.workspace, scratch.workspace_bytes, scratch.counters, scratch.num_counters, &d,
+                            static_cast<float>(scale),
                              fmt, static_cast<float>(k_scale), static_cast<float>(v_scale),
                              static_cast<int>(num_splits), stream);
   TORCH_CHECK(st == PAD_OK, "pa_decode: ", pad_status_string(st));

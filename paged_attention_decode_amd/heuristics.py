@@ -38,6 +38,8 @@ OVERSUBSCRIBE_SPLITS = 4   # items per unit on an oversubscribed grid, at least,
 OVERSUBSCRIBE_GROUPS_PER_CU = 8  # and at least this many workgroups per CU
 PLAN_MAX_BATCH = 256       # largest batch the in-kernel planner handles
 TWO_LEVEL_SPLITS = 48      # units with more splits merge in two levels (groups of 16)
+RANGE_MAX_BATCH = 512      # largest batch a range launch takes
+RANGE_ROW_BYTES = 3 << 19  # fewest fp16 K/V bytes of a full table row in one head group
 
 
 @dataclass(frozen=True)
@@ -76,9 +78,57 @@ def plan(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, page_si
          num_splits: int = 0, num_cus: int = 256, engine: int = 0, csr: bool = False, kv_bytes: int = 2) -> Plan:
     """Same result as ``pad_decode_plan`` (``pad_decode_plan_csr`` with ``csr``) for valid arguments.
 
+    Where the launch takes the range kernel (``range_launch``), its waves, and
+    scratch for both it and the per-unit kernel, which a launch with less
+    scratch runs.
+
     ``kv_bytes=1`` gives the plan of an fp8-cache launch (pad_decode_launch_kv8): the same splits and
     scratch except where the fp16 plan is an oversubscribed grid (fp8 takes the 4-item grid from one
     unit per CU up only: never more scratch), 8-wave workgroups for its 128-byte rows at head_dim 128."""
+    p = plan_units(batch, num_q_heads, num_kv_heads, head_dim, page_size, max_pages, num_splits, num_cus, engine,
+                   csr, kv_bytes)
+    r = None
+    if num_splits == 0 and engine == 0:
+        r = range_launch(batch, num_q_heads, num_kv_heads, head_dim, page_size, max_pages, num_cus, csr, kv_bytes)
+    if r is None:
+        return p
+    groups, heads, waves = r
+    rows = 2 * groups * heads * (num_q_heads // num_kv_heads)
+    return Plan(p.num_splits, p.pages_per_split, waves, False,
+                max(p.workspace_bytes, 256 + rows * head_dim * 4 + rows * 8),
+                max(p.counters, batch * num_kv_heads // heads + 2 * groups))
+
+
+def range_launch(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, page_size: int, max_pages: int,
+                 num_cus: int = 256, csr: bool = False, kv_bytes: int = 2) -> tuple[int, int, int] | None:
+    """(workgroups, kv heads per workgroup, waves) of a heuristic launch that takes the range kernel, or None.
+
+    Bandwidth-bound shapes with units as the oversubscribed grid takes them
+    and batch <= RANGE_MAX_BATCH, except two kv heads and short table rows."""
+    if num_cus <= 0:
+        num_cus = 256
+    units = batch * num_kv_heads
+    mp = pages_per_seq(batch, max_pages, csr)
+    if batch <= 0 or batch > RANGE_MAX_BATCH or num_kv_heads == 2:
+        return None
+    latency_bound = units * _cdiv(mp * page_size, BLOCK_TOKENS) <= 16 * num_cus
+    if units * 4 <= num_cus or units * 2 == num_cus or latency_bound:
+        return None
+    heads = 4 if num_kv_heads % 4 == 0 else 2 if num_kv_heads % 2 == 0 else 1
+    if mp * page_size * head_dim * 4 * heads < RANGE_ROW_BYTES:
+        return None
+    if batch * (2 * max_pages + 4096) > (1 << 30) // num_kv_heads:
+        return None
+    p = plan_units(batch, num_q_heads, num_kv_heads, head_dim, page_size, max_pages, 0, num_cus, 0, csr)
+    groups = min(units * p.num_splits, num_cus)
+    if batch > 2 * groups:
+        return None
+    return groups, heads, MAX_WAVES if head_dim * kv_bytes <= 128 else MAX_WAVES // 2
+
+
+def plan_units(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, page_size: int, max_pages: int,
+               num_splits: int = 0, num_cus: int = 256, engine: int = 0, csr: bool = False, kv_bytes: int = 2) -> Plan:
+    """The per-unit kernel's plan."""
     if num_cus <= 0:
         num_cus = 256
     gqa = num_q_heads // num_kv_heads
@@ -110,8 +160,8 @@ def plan(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, page_si
         cap = max(cap, 1)
         want = max(min(want, cap, MAX_SPLITS), 1)
         if csr:  # never more splits (scratch) than the dense plan of the same dims
-            want = min(want, plan(batch, num_q_heads, num_kv_heads, head_dim, page_size, max_pages, 0, num_cus,
-                                  engine).num_splits)
+            want = min(want, plan_units(batch, num_q_heads, num_kv_heads, head_dim, page_size, max_pages, 0,
+                                        num_cus, engine).num_splits)
         pps = _cdiv(mp, want)
         s = _cdiv(mp, pps)
     nw = _cdiv(pps * page_size, BLOCK_TOKENS)

@@ -1,7 +1,7 @@
 """Register and scratch use of every decode-kernel instantiation, from the compiler.
 
-Compiles ``csrc/pa_decode.hip`` for gfx950 (device code only, the product
-flags of ``build.py``) with ``-Rpass-analysis=kernel-resource-usage`` and
+Compiles ``csrc/pa_decode.hip`` and ``csrc/pa_range.hip`` for gfx950 (device
+code only, the product flags of ``build.py``) with ``-Rpass-analysis=kernel-resource-usage`` and
 parses the remarks: per kernel VGPRs, AGPRs, SGPRs, scratch bytes per lane,
 SGPR and VGPR spill counts, occupancy (waves per SIMD) and static LDS.
 
@@ -18,6 +18,7 @@ import argparse
 import os
 import re
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 
 from . import build
 
@@ -38,7 +39,8 @@ def _demangle_args(name: str) -> str:
     # a fifth argument of 1-5 is printed as e4m3fn / e5m2 (fp8 caches, fp16 q),
     # bf16, e4m3fn/bf16 / e5m2/bf16 (fp8 caches, bfloat16 q).
     args = re.findall(r"Li(\d+)E", name)
-    if len(args) == 5:
+    # pad_range_kernel: <head_dim, block mode> and the format
+    if len(args) in (3, 5):
         kvf = args.pop()
         if kvf != "0":
             args.append({"1": "e4m3fn", "2": "e5m2", "3": "bf16", "4": "e4m3fn/bf16",
@@ -47,11 +49,16 @@ def _demangle_args(name: str) -> str:
 
 
 def collect(defines: tuple[str, ...] = ()) -> list[dict]:
-    """One dict per kernel of pa_decode.hip (name, template args and FIELDS)."""
+    """One dict per kernel of the library (name, template args and FIELDS)."""
+    with ThreadPoolExecutor(max_workers=len(build.CAPI_SOURCES)) as pool:
+        return sum(pool.map(lambda name: _collect_source(name, defines), build.CAPI_SOURCES), [])
+
+
+def _collect_source(name: str, defines: tuple[str, ...]) -> list[dict]:
     hipcc = os.path.join(build.ROCM, "bin", "hipcc")
     flags = [f for f in build.HIP_FLAGS if f != "-shared"]
     cmd = [hipcc, *flags, *[f"-D{d}" for d in defines], f"-I{build.INCLUDE}", "--cuda-device-only", "-c",
-           os.path.join(build.CSRC, "pa_decode.hip"), "-o", os.devnull, "-Rpass-analysis=kernel-resource-usage"]
+           os.path.join(build.CSRC, name + ".hip"), "-o", os.devnull, "-Rpass-analysis=kernel-resource-usage"]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
         raise RuntimeError("compile failed:\n" + proc.stdout[-4000:])
@@ -72,7 +79,8 @@ def table(rows: list[dict]) -> str:
     out = [f"{'kernel':22s} {'template':18s} {'VGPR':>4s} {'AGPR':>4s} {'SGPR':>4s} {'scratch':>7s} "
            f"{'sgpr_spill':>10s} {'vgpr_spill':>10s} {'waves/SIMD':>10s} {'LDS':>5s}"]
     for r in rows:
-        kern = next((k for k in ("pad_phase1_kernel", "pad_plan_kernel", "pad_zero_i32_kernel") if k in r["name"]), r["name"][:22])
+        kern = next((k for k in ("pad_phase1_kernel", "pad_range_kernel", "pad_plan_kernel",
+                                 "pad_range_plan_kernel", "pad_zero_i32_kernel") if k in r["name"]), r["name"][:22])
         tmpl = r["template"] if r["template"].startswith("<") else "-"
         out.append(f"{kern:22s} {tmpl:18s} {r.get('vgpr', 0):4d} {r.get('agpr', 0):4d} "
                    f"{r.get('sgpr', 0):4d} {r.get('scratch', 0):7d} {r.get('sgpr_spill', 0):10d} "
@@ -86,9 +94,11 @@ def main() -> None:
     a = p.parse_args()
     rows = collect(tuple(a.define))
     print(table(rows))
-    phase1 = [r for r in rows if "pad_phase1_kernel" in r["name"]]
-    spilled = [r for r in phase1 if r.get("vgpr_spill", 0) or r.get("scratch", 0)]
-    print(f"\n{len(phase1)} pad_phase1_kernel instantiations; {len(spilled)} with VGPR spills or scratch")
+    print()
+    for kernel in ("pad_phase1_kernel", "pad_range_kernel"):
+        mine = [r for r in rows if kernel in r["name"]]
+        spilled = [r for r in mine if r.get("vgpr_spill", 0) or r.get("scratch", 0)]
+        print(f"{len(mine)} {kernel} instantiations; {len(spilled)} with VGPR spills or scratch")
 
 
 if __name__ == "__main__":

@@ -1,0 +1,160 @@
+"""The range kernel (csrc/pa_range.hip): equal page ranges, head groups.
+
+GPU: every element format, page-size mode, head_dim and head-group size that
+a launch takes to it, at the edges of its ranges (ragged lengths with empty
+sequences at both ends, one-token sequences, lengths around page and block
+ends; equal lengths cut alike, in whole units per workgroup, and in whole
+units with batches past one register of the table), through the dense table,
+the CSR index and a work list, against the fp32 oracle (bfloat16 and fp8 with
+bfloat16 q at the bfloat16 tolerance).  A launch with the per-unit kernel's
+scratch runs that kernel.
+
+CPU: which shapes take it, and that its scratch is in the plan's.
+"""
+
+from __future__ import annotations
+
+import ctypes
+import random
+
+import pytest
+import torch
+
+from oracle.reference import decode_fp16_protocol
+from paged_attention_decode_amd import _native, heuristics
+from tests.helpers import make_cache, shuffled_table
+
+DTYPES = {"fp16": torch.float16, "bf16": torch.bfloat16, "e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}
+
+
+def _lens(kind, batch, cap, ps, seed):
+    rng = random.Random(seed)
+    if kind == "equal":
+        return [cap] * batch
+    if kind == "equal_pages":  # the same page count, last pages partly filled
+        return [cap - rng.randint(0, ps - 1) for _ in range(batch)]
+    lens = [rng.choice([rng.randint(1, cap), rng.randint(1, min(cap, 40)), cap]) for _ in range(batch)]
+    lens[0] = lens[-1] = lens[batch // 2] = lens[batch // 2 + 1] = 0
+    lens[1], lens[2], lens[3] = 1, cap, min(cap, 17)
+    return lens
+
+
+CASES = [
+    # (lengths, batch, kv heads, group, head_dim, page size, table tokens, q, kv)
+    ("ragged", 40, 4, 4, 128, 16, 2048, "fp16", "fp16"),
+    ("ragged", 40, 4, 3, 128, 32, 2048, "bf16", "bf16"),
+    ("ragged", 70, 8, 2, 128, 1, 1024, "bf16", "bf16"),
+    ("ragged", 40, 4, 4, 128, 2, 2048, "fp16", "fp16"),
+    ("ragged", 40, 4, 4, 128, 4, 2048, "fp16", "e5m2"),
+    ("ragged", 40, 4, 4, 128, 8, 2048, "bf16", "e4m3"),
+    ("ragged", 40, 4, 4, 128, 12, 2048, "fp16", "e4m3"),
+    ("ragged", 40, 8, 1, 128, 3, 1000, "fp16", "fp16"),
+    ("ragged", 24, 8, 4, 64, 16, 2048, "fp16", "fp16"),
+    ("ragged", 24, 8, 16, 64, 24, 2048, "bf16", "e5m2"),
+    ("ragged", 24, 8, 3, 96, 16, 1500, "fp16", "fp16"),
+    ("ragged", 40, 4, 4, 32, 16, 4096, "bf16", "bf16"),
+    ("ragged", 33, 4, 16, 256, 16, 1024, "bf16", "bf16"),
+    ("ragged", 33, 4, 2, 256, 5, 1024, "fp16", "e4m3"),
+    ("ragged", 70, 6, 2, 128, 16, 2048, "fp16", "fp16"),  # two kv heads per workgroup
+    ("ragged", 300, 1, 8, 128, 16, 4096, "fp16", "fp16"),  # past the per-unit planner's batch
+    ("ragged", 512, 1, 2, 128, 64, 3200, "fp16", "fp16"),
+    ("ragged", 140, 1, 16, 256, 1, 2048, "fp16", "fp16"),
+    ("equal", 17, 8, 4, 128, 16, 1040, "fp16", "fp16"),
+    ("equal_pages", 33, 4, 8, 128, 16, 2048, "bf16", "e4m3"),
+    ("equal", 140, 8, 1, 64, 16, 2048, "fp16", "fp16"),  # 280 head groups: two whole units per workgroup
+    ("equal_pages", 260, 4, 1, 32, 8, 3072, "fp16", "fp16"),
+]
+
+
+def _inputs(case):
+    kind, batch, hkv, group, d, ps, room, qt, kvt = case
+    lens = _lens(kind, batch, room, ps, seed=batch + d)
+    width = -(-room // ps)
+    used = max(-(-n // ps) for n in lens)
+    bt, num_pages = shuffled_table(lens, ps, spare_pages=2, extra_cols=width - used, seed=d)
+    k, v = make_cache(num_pages, ps, hkv, d, seed=batch)
+    q = torch.randn(batch, hkv * group, d, generator=torch.Generator().manual_seed(ps)).to(DTYPES[qt])
+    k, v = k.to(DTYPES[kvt]), v.to(DTYPES[kvt])
+    return lens, q, k, v, bt, torch.tensor(lens, dtype=torch.int32)
+
+
+def _check(out, expected, qt):
+    # bfloat16: P and the output are rounded to 8 bits, as in tests/test_bf16.py
+    tol = 2e-3 if qt == "fp16" else 1e-2
+    got = out.float().cpu()
+    assert torch.isfinite(got).all()
+    assert torch.allclose(got, expected, rtol=tol, atol=tol), (got - expected).abs().max().item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
+def test_range_kernel_against_oracle(case):
+    import paged_attention_decode_amd as pad
+
+    kind, batch, hkv, group, d, ps, room, qt, kvt = case
+    lens, q, k, v, bt, sl = _inputs(case)
+    hq = hkv * group
+    assert heuristics.range_launch(batch, hq, hkv, d, ps, bt.shape[1]) is not None
+    expected = decode_fp16_protocol(q.float(), k.float(), v.float(), bt, sl)
+    qd, kd, vd, btd, sld = q.cuda(), k.cuda(), v.cuda(), bt.cuda(), sl.cuda()
+    fp8 = kvt in ("e4m3", "e5m2")
+    dense = pad.paged_attention_decode_fp8 if fp8 else pad.paged_attention_decode_ex
+    out = dense(qd, kd, vd, btd, sld)
+    _check(out, expected, qt)
+    assert torch.equal(out, dense(qd, kd, vd, btd, sld))  # the same bits again
+    w = pad.BatchDecodeWrapper()
+    types = dict(q_data_type=DTYPES[qt], kv_data_type=DTYPES[kvt])
+    w.plan_block_table(btd, sld, hq, hkv, d, ps, **types)
+    assert torch.equal(out, w.run(qd, (kd, vd)))
+    indptr, indices, last = pad.paged_kv_indices(btd, sld, ps)
+    csr = pad.paged_attention_decode_csr(qd, kd, vd, indptr, indices, last)
+    _check(csr, expected, qt)
+    w.plan(indptr, indices, last, hq, hkv, d, ps, **types)
+    assert torch.equal(csr, w.run(qd, (kd, vd)))
+
+
+@pytest.mark.gpu
+def test_least_scratch_runs_the_per_unit_kernel():
+    lib = _native.capi()
+    case = CASES[0]
+    lens, q, k, v, bt, sl = _inputs(case)
+    expected = decode_fp16_protocol(q.float(), k.float(), v.float(), bt, sl)
+    qd, kd, vd, btd, sld = q.cuda(), k.cuda(), v.cuda(), bt.cuda(), sl.cuda()
+    out = torch.empty_like(qd)
+    dm = _native.dims_for(qd, kd, vd, btd, sld, out)
+    full, least, n, least_n = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_int64(), ctypes.c_int64()
+    assert lib.pad_decode_workspace_bytes(ctypes.byref(dm), 0, 0, ctypes.byref(full)) == 0
+    assert lib.pad_decode_counters_needed(ctypes.byref(dm), 0, 0, ctypes.byref(n)) == 0
+    assert lib.pad_decode_least_scratch(ctypes.byref(dm), 0, 0, 0, ctypes.byref(least), ctypes.byref(least_n)) == 0
+    assert least.value <= full.value and least_n.value <= n.value
+    counters = torch.zeros(n.value, dtype=torch.int32, device="cuda")
+    ws = torch.empty(full.value, dtype=torch.uint8, device="cuda")
+    for nbytes in (full.value, least.value):
+        out.zero_()
+        st = lib.pad_decode_launch(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), btd.data_ptr(), sld.data_ptr(),
+                                   out.data_ptr(), ws.data_ptr(), nbytes, counters.data_ptr(), n.value,
+                                   ctypes.byref(dm), ctypes.c_float(128 ** -0.5), 0,
+                                   torch.cuda.current_stream().cuda_stream)
+        assert st == 0
+        torch.cuda.synchronize()
+        _check(out, expected, "fp16")
+        assert int(counters.abs().sum()) == 0
+
+
+def test_shapes_that_take_the_range_kernel():
+    r = heuristics.range_launch
+    assert r(256, 64, 8, 128, 16, 2048) == (256, 4, 4)
+    assert r(64, 32, 8, 128, 16, 512, kv_bytes=1) == (256, 4, 8)
+    assert r(300, 8, 1, 128, 16, 256) == (256, 1, 4)
+    assert r(70, 12, 6, 128, 16, 128) == (256, 2, 4)
+    assert r(64, 12, 2, 128, 16, 256) is None  # two kv heads
+    assert r(1, 32, 8, 128, 16, 8192) is None  # few units: the per-unit kernel's shorter merge
+    assert r(200, 64, 8, 128, 16, 8) is None  # short rows
+    assert r(513, 8, 1, 128, 16, 4096) is None
+    for batch, hq, hkv, d, ps, pages in ((256, 64, 8, 128, 16, 2048), (300, 8, 1, 128, 16, 256), (33, 64, 4, 256, 16, 64)):
+        p = heuristics.plan(batch, hq, hkv, d, ps, pages)
+        u = heuristics.plan_units(batch, hq, hkv, d, ps, pages)
+        groups, heads, _ = r(batch, hq, hkv, d, ps, pages)
+        rows = 2 * groups * heads * (hq // hkv)
+        assert p.workspace_bytes >= max(u.workspace_bytes, rows * (d * 4 + 8)) and not p.single_pass
+        assert p.counters >= max(u.counters, batch * hkv // heads + 2 * groups)

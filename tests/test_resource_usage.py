@@ -17,8 +17,13 @@ pytestmark = pytest.mark.skipif(not os.path.exists(os.path.join(build.ROCM, "bin
 
 
 @pytest.fixture(scope="module")
-def rows():
-    return [r for r in resource_usage.collect() if "pad_phase1_kernel" in r["name"]]
+def kernels():
+    return resource_usage.collect()
+
+
+@pytest.fixture(scope="module")
+def rows(kernels):
+    return [r for r in kernels if "pad_phase1_kernel" in r["name"]]
 
 
 def test_every_instantiation_is_reported(rows):
@@ -46,3 +51,10 @@ def test_headline_kernel_fits_three_waves_per_simd(rows):
     # hold three 4-wave workgroups when the grid oversubscribes it (C5).
     r = next(r for r in rows if r["template"] == "<128, 1, 0, 0>")
     assert r["occupancy"] >= 3 and r["vgpr"] + r.get("agpr", 0) <= 168
+
+
+def test_range_kernel_has_no_scratch_memory(kernels):
+    rows = [r for r in kernels if "pad_range_kernel" in r["name"]]
+    # head_dims 32-256 x 6 block modes in fp16 and bfloat16, 64-256 in the four fp8 forms
+    assert len(rows) == 2 * 5 * 6 + 4 * 3 * 6
+    assert not [r["template"] for r in rows if r.get("scratch", 0)]
