@@ -1333,6 +1333,7 @@ struct RangeShape {
   int nh_shift;  // log2 of the kv heads per workgroup
   int nw;        // waves per workgroup
   int unit_extra;  // positions a unit counts beyond its pages
+  int min_chunk;   // pages per range, at least
   size_t workspace_bytes;
   int64_t counters;
 };
@@ -1466,9 +1467,9 @@ static int plan_units(const pad_decode_dims* d, int num_splits, int num_cus, int
   return PAD_OK;
 }
 
-// Fewest 16-token blocks per range: what a workgroup streams against its fixed
-// costs (q and the first K/V loads, merge, partial).
-constexpr int kRangeMinBlocks = 16;
+// Fewest K/V bytes per range: what a workgroup streams against its fixed costs
+// (q and the first K/V loads, merge, partial).
+constexpr int64_t kRangeMinBytes = 192 * 1024;
 // What a workgroup streams in the time it takes from one unit of its range to
 // the next: its waves' states merged and written, the next unit's first
 // loads.  64 x [1, 8192] tokens of 32/8 heads (fp8) with 0 / 40 / 80 / 160 /
@@ -1487,6 +1488,12 @@ constexpr int64_t kRangeUnitBytes = 160 * 1024;
 // sequences, rows of 1024 and 4096 tokens) still gain, 27.2 against 35.1 and
 // 39.4 against 57.5 us, as the per-unit grid is then oversubscribed in vain.
 constexpr int64_t kRangeRowBytes = 3 << 19;
+// Fewest fp16 K/V bytes of all rows: below, the per-unit grid's shorter way to
+// the first load and its smaller merges count for more (us per call, range
+// against per unit: 3 sequences, 38 MB of 32/32 heads, 16.0 against 14.5; 11,
+// 63 MB of 32/8, 21.1 against 19.4; 10, 132 MB of 64/8, 19.8 against 14.6; at
+// 162 MB, 8 of 32/32 with fp8 caches, 16.8 against 38.6).
+constexpr int64_t kRangeCallBytes = 1 << 27;
 
 // Takes the calls that the per-unit kernel plans on an oversubscribed grid
 // (more units than a few per CU's worth of splits would balance, see
@@ -1501,7 +1508,7 @@ constexpr int64_t kRangeRowBytes = 3 << 19;
 // 4 x 8192: 26.3 against 28.6-32 us).
 static RangeShape range_shape(const pad_decode_dims* d, int num_splits, int num_cus, int engine, bool csr,
                               int kv_bytes) {
-  RangeShape r = {0, 0, 0, 0, 0, 0};
+  RangeShape r = {0, 0, 0, 0, 0, 0, 0};
 #ifdef PAD_TIMELINE
   return r;  // the phase stamps are the per-unit kernel's
 #endif
@@ -1512,7 +1519,7 @@ static RangeShape range_shape(const pad_decode_dims* d, int num_splits, int num_
   r.nh_shift = d->num_kv_heads % 4 == 0 ? 2 : (d->num_kv_heads % 2 == 0 ? 1 : 0);
   const int64_t page_bytes = ((int64_t)d->page_size * d->head_dim * kv_bytes * 2) << r.nh_shift;
   const int64_t row_bytes = plan_pages_per_seq(d, csr) * (((int64_t)d->page_size * d->head_dim * 4) << r.nh_shift);
-  if (row_bytes < kRangeRowBytes) return r;
+  if (row_bytes < kRangeRowBytes || (units >> r.nh_shift) * row_bytes < kRangeCallBytes) return r;
   // Positions are counted in 32 bits (twice the pages at most, and unit_extra).
   if (d->batch * (2 * (int64_t)d->max_pages + 4096) > (1 << 30) / d->num_kv_heads) return r;
   // A work list holds a record per workgroup and two sequences per record.
@@ -1527,6 +1534,7 @@ static RangeShape range_shape(const pad_decode_dims* d, int num_splits, int num_
   // 24 x [1, 4096]: 22.5 and 23.1 us).
   r.nw = d->head_dim * kv_bytes <= 128 ? kMaxWaves : kMaxWaves / 2;
   r.unit_extra = ceil_div(kRangeUnitBytes, page_bytes);
+  r.min_chunk = ceil_div(kRangeMinBytes, page_bytes);
   r.workspace_bytes = range_layout(d, r, nullptr, nullptr, nullptr);
   r.counters = (units >> r.nh_shift) + 2 * (int64_t)groups;
   return r;
@@ -1788,7 +1796,7 @@ static int setup_launch(const void* q, const void* k, const void* v, const int32
     a.hkv = d->num_kv_heads >> rs.nh_shift;
     a.num_splits = a.pps = a.pair_heads = 0;
     a.balance = 1;
-    a.min_chunk = ceil_div(kRangeMinBlocks * kBlockTokens, d->page_size);
+    a.min_chunk = rs.min_chunk;
     a.unit_extra = rs.unit_extra;
   }
   a.wl_key = plan_key(a);

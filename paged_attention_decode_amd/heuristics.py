@@ -40,6 +40,7 @@ PLAN_MAX_BATCH = 256       # largest batch the in-kernel planner handles
 TWO_LEVEL_SPLITS = 48      # units with more splits merge in two levels (groups of 16)
 RANGE_MAX_BATCH = 512      # largest batch a range launch takes
 RANGE_ROW_BYTES = 3 << 19  # fewest fp16 K/V bytes of a full table row in one head group
+RANGE_CALL_BYTES = 1 << 27  # and of all rows and groups
 
 
 @dataclass(frozen=True)
@@ -115,7 +116,8 @@ def range_launch(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int,
     if units * 4 <= num_cus or units * 2 == num_cus or latency_bound:
         return None
     heads = 4 if num_kv_heads % 4 == 0 else 2 if num_kv_heads % 2 == 0 else 1
-    if mp * page_size * head_dim * 4 * heads < RANGE_ROW_BYTES:
+    row_bytes = mp * page_size * head_dim * 4 * heads
+    if row_bytes < RANGE_ROW_BYTES or units // heads * row_bytes < RANGE_CALL_BYTES:
         return None
     if batch * (2 * max_pages + 4096) > (1 << 30) // num_kv_heads:
         return None

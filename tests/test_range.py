@@ -49,17 +49,17 @@ CASES = [
     ("ragged", 40, 4, 4, 128, 8, 2048, "bf16", "e4m3"),
     ("ragged", 40, 4, 4, 128, 12, 2048, "fp16", "e4m3"),
     ("ragged", 40, 8, 1, 128, 3, 1000, "fp16", "fp16"),
-    ("ragged", 24, 8, 4, 64, 16, 2048, "fp16", "fp16"),
-    ("ragged", 24, 8, 16, 64, 24, 2048, "bf16", "e5m2"),
-    ("ragged", 24, 8, 3, 96, 16, 1500, "fp16", "fp16"),
-    ("ragged", 40, 4, 4, 32, 16, 4096, "bf16", "bf16"),
+    ("ragged", 40, 8, 4, 64, 16, 2048, "fp16", "fp16"),
+    ("ragged", 40, 8, 16, 64, 24, 2048, "bf16", "e5m2"),
+    ("ragged", 40, 8, 3, 96, 16, 1500, "fp16", "fp16"),
+    ("ragged", 70, 4, 4, 32, 16, 4096, "bf16", "bf16"),
     ("ragged", 33, 4, 16, 256, 16, 1024, "bf16", "bf16"),
     ("ragged", 33, 4, 2, 256, 5, 1024, "fp16", "e4m3"),
     ("ragged", 70, 6, 2, 128, 16, 2048, "fp16", "fp16"),  # two kv heads per workgroup
     ("ragged", 300, 1, 8, 128, 16, 4096, "fp16", "fp16"),  # past the per-unit planner's batch
     ("ragged", 512, 1, 2, 128, 64, 3200, "fp16", "fp16"),
     ("ragged", 140, 1, 16, 256, 1, 2048, "fp16", "fp16"),
-    ("equal", 17, 8, 4, 128, 16, 1040, "fp16", "fp16"),
+    ("equal", 40, 8, 4, 128, 16, 1040, "fp16", "fp16"),
     ("equal_pages", 33, 4, 8, 128, 16, 2048, "bf16", "e4m3"),
     ("equal", 140, 8, 1, 64, 16, 2048, "fp16", "fp16"),  # 280 head groups: two whole units per workgroup
     ("equal_pages", 260, 4, 1, 32, 8, 3072, "fp16", "fp16"),
@@ -150,6 +150,7 @@ def test_shapes_that_take_the_range_kernel():
     assert r(64, 12, 2, 128, 16, 256) is None  # two kv heads
     assert r(1, 32, 8, 128, 16, 8192) is None  # few units: the per-unit kernel's shorter merge
     assert r(200, 64, 8, 128, 16, 8) is None  # short rows
+    assert r(43, 32, 8, 64, 16, 96) == (256, 4, 8) and r(42, 32, 8, 64, 16, 96) is None  # few bytes in all
     assert r(513, 8, 1, 128, 16, 4096) is None
     for batch, hq, hkv, d, ps, pages in ((256, 64, 8, 128, 16, 2048), (300, 8, 1, 128, 16, 256), (33, 64, 4, 256, 16, 64)):
         p = heuristics.plan(batch, hq, hkv, d, ps, pages)
