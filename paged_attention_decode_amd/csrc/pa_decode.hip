@@ -1138,6 +1138,135 @@ void pad_phase1_kernel(const Phase1Args a) {
   PAD_TL(lin, PAD_TL_PUBLISHED);
   int tl_flags = 0;
   (void)tl_flags;
+  // GQA_T == 1 marks the MFMA kernels that hold the shared fold: its registers
+  // would cost the others occupancy (a d64 grid of several workgroups per CU
+  // 98.4 -> 106.9 us).
+  if (ENGINE == 0 && GQA_T == 1 && nsplit * total4 >= kSharedFoldElements &&
+      nsplit <= max(kTwoLevelSplits, total4 / 16)) {
+    // Shared fold: every workgroup of the unit folds one slice of the output,
+    // where the last arrival alone would read 256 KB or more with one
+    // workgroup's loads in flight (8 x 8192 tokens, 16/1 heads of 256, 32
+    // splits: 10.2 us from the last arrival to the output, 4.4 us shared; the
+    // call 26.0 us at its 16 splits before, 21.0 us now; 8 x 16384 of 16/1 at
+    // 128 22.9 -> 19.8 us).
+    //
+    // counter = arrivals + departures << 16, on a line of the unit's own (its
+    // group counters, which it leaves unused: with all units' polls on one
+    // line the arrivals alone took 11 us).  A workgroup arrives, waits until
+    // all have, departs, and folds its slice; the last to depart resets the
+    // counter.  Waiting is bounded, as nothing says that all workgroups of a
+    // unit run at once: one out of polls departs early, and the departures
+    // that the last arrival finds tell it to fold the whole unit itself
+    // (workgroups that fold their own slice as well write the same bits).
+    // Without a bound of the streaming time of a split, the short last split
+    // of a sequence gives up and the whole fold falls to one workgroup.
+    __shared__ int s_fold;
+    int* fold_counter = a.counters + (int64_t)a.batch * a.hkv + it.slot0;
+    int departed = 0;
+    if (threadIdx.x == 0) {
+      const int before = atomicAdd(fold_counter, 1);
+      int fold = 0;  // 1: own slice, 2: the whole unit
+      if ((before & 0xffff) == nsplit - 1) {
+        fold = before >> 16 ? 2 : 1;
+      } else {
+        for (int i = a.fold_polls; i > 0 && !fold; --i) {
+          __builtin_amdgcn_s_sleep(8);
+          fold = (__hip_atomic_load(fold_counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xffff) == nsplit;
+        }
+      }
+      if (!fold) {
+        departed = atomicAdd(fold_counter, 1 << 16);
+        fold = (departed & 0xffff) == nsplit ? 3 : 0;  // 3: as 1 (the last one arrived in between)
+      }
+      s_fold = fold;
+    }
+    __syncthreads();
+    PAD_TL(lin, PAD_TL_ARRIVED);
+    const int fold = s_fold;
+    if (fold == 0) {
+      PAD_TL_NOTE(g, 0);
+      PAD_TL(lin, PAD_TL_EXIT);
+      return;
+    }
+    if (threadIdx.x == 0 && fold != 3) departed = atomicAdd(fold_counter, 1 << 16);
+    // An element's splits fold in runs of `cnt`, a thread each, and the runs'
+    // states through LDS in order; the whole-unit fold keeps that order.
+    const int nt = nw * 64;
+    const int per = (total4 + nsplit - 1) / nsplit;
+    int runs = min((nsplit + 3) / 4, max(1, nt / per));
+    const int cnt = (nsplit + runs - 1) / runs;
+    runs = (nsplit + cnt - 1) / cnt;
+    const int hi = min((my_split + 1) * per, total4);
+    const int span = min(per, nt / runs);
+    f4_t* run_o = reinterpret_cast<f4_t*>(sm_ml);  // [runs][span], then the (m, l) pairs
+    float2* run_ml = reinterpret_cast<float2*>(run_o + nt);
+    for (int e0 = fold == 2 ? threadIdx.x : my_split * per; e0 < (fold == 2 ? total4 : hi); e0 += fold == 2 ? nt : span) {
+      float m = kNegInf, l = 0.f;
+      f4_t acc = (f4_t)0.f;
+      int e = e0;
+      if (fold == 2) {
+        const int row = e / (D / 4);
+        const int col = (e - row * (D / 4)) * 4;
+        for (int r0 = 0; r0 < runs; r0 += 2) {
+          MergeBatch<4> p[2];  // the first 4 entries of two runs
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            p[i].load_below(o_rsrc, ml_rsrc, (r0 + i) * cnt, min((r0 + i + 1) * cnt, nsplit), gqa, row, col, D);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int first = (r0 + i) * cnt;
+            const int end = min(first + cnt, nsplit);
+            if (first < end) {
+              float mr = kNegInf, lr = 0.f;
+              f4_t ar = (f4_t)0.f;
+              p[i].fold(first, end, mr, lr, ar);
+              for (int sp0 = first + 4; sp0 < end; sp0 += 4) {
+                MergeBatch<4> q;
+                q.load_below(o_rsrc, ml_rsrc, sp0, end, gqa, row, col, D);
+                q.fold(sp0, end, mr, lr, ar);
+              }
+              fold_state(mr, lr, ar, m, l, acc);
+            }
+          }
+        }
+      } else {
+        const int run = threadIdx.x / span;
+        e = e0 + threadIdx.x - run * span;
+        if (run < runs && e < hi) {
+          const int row = e / (D / 4);
+          const int col = (e - row * (D / 4)) * 4;
+          fold_run(o_rsrc, ml_rsrc, run * cnt, min((run + 1) * cnt, nsplit), gqa, row, col, D, m, l, acc);
+          run_o[threadIdx.x] = acc;
+          run_ml[threadIdx.x] = make_float2(m, l);
+        }
+        __syncthreads();
+        if (run > 0 || e >= hi) e = total4;
+        m = kNegInf;
+        l = 0.f;
+        acc = (f4_t)0.f;
+        if (e < total4)
+          for (int r = 0; r < runs; ++r) {
+            const float2 ml = run_ml[r * span + threadIdx.x];
+            fold_state(ml.x, ml.y, run_o[r * span + threadIdx.x], m, l, acc);
+          }
+        __syncthreads();
+      }
+      if (e < total4) {
+        const int row = e / (D / 4);
+        const int col = (e - row * (D / 4)) * 4;
+        const float inv = (kv_is_fp8<KVF>() ? a.v_fix : 1.f) / l;
+        h4_t hv;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) hv[i] = round16<KVF>(acc[i] * inv);
+        *reinterpret_cast<h4_t*>(out_bh + (int64_t)row * a.soh + col) = hv;
+      }
+    }
+    if (threadIdx.x == 0 && (departed >> 16) == nsplit - 1) atomicExch(fold_counter, 0);
+    PAD_TL(lin, PAD_TL_MERGED);
+    PAD_TL_NOTE(g, PAD_TL_F_MERGER);
+    PAD_TL(lin, PAD_TL_EXIT);
+    return;
+  }
   if (nsplit > kTwoLevelSplits) {
     const int grp0 = my_split & ~15;  // first split of this group
     const int gsize = min(16, nsplit - grp0);
@@ -1393,7 +1522,13 @@ static int plan_units(const pad_decode_dims* d, int num_splits, int num_cus, int
     // batch 20 20.8 against 19.2 us with 6; batch 5 12.3 against 11.7 us with
     // 12), while smaller steps lose to the longer merge (batch 7, 8 -> 9
     // splits, and batch 12, 8 -> 10: +2%).
-    const int64_t max_groups = latency_bound ? num_cus / 2 : num_cus;
+    // A unit that shares its fold (kSharedFoldElements) at one workgroup per
+    // CU pays no longer merge for more splits and takes all CUs (8 x 8192,
+    // 16/1 heads of 256: 21.0 us against 23.4 us on half).
+    const int64_t s_all = num_cus / units;
+    const bool shared_fold = engine == 0 && s_all <= kTwoLevelSplits &&
+                             s_all * gqa * (d->head_dim / 4) >= kSharedFoldElements;
+    const int64_t max_groups = latency_bound && !shared_fold ? num_cus / 2 : num_cus;
     int64_t s_want = 1;
     while (s_want * 2 * units <= max_groups) s_want *= 2;
     const int64_t s_fit = max_groups / units;
@@ -1576,6 +1711,8 @@ static int device_cus(int* out) {
 
 template <int D, int MODE, int ENGINE, int GQA_T, int KVF = kKvF16>
 static hipError_t launch_p1(const Phase1Args& a, dim3 grid, int nw, size_t lds, hipStream_t st) {
+  if constexpr (ENGINE == 0 && GQA_T == 0 && D >= 128)  // smaller rows never reach kSharedFoldElements
+    if (a.fold_polls > 0) return launch_p1<D, MODE, 0, 1, KVF>(a, grid, nw, lds, st);
   hipLaunchKernelGGL((pad_phase1_kernel<D, MODE, ENGINE, GQA_T, KVF>), grid, dim3(nw * 64), lds, st, a);
   return hipGetLastError();
 }
@@ -1783,6 +1920,15 @@ static int setup_launch(const void* q, const void* k, const void* v, const int32
     if ((1 << sh) == d->page_size) a.ps_shift = sh;
   a.scale_log2 = scale * kLog2e;
   a.v_fix = 1.0f;
+  a.fold_polls = 0;
+  // The shared fold waits for a unit's other workgroups: only where the whole
+  // grid can run at once, each unit has group counters, and a unit can get
+  // the splits (the planner may give one more than S).
+  const int total4 = gqa * (d->head_dim / 4);
+  const int most_splits = a.balance ? (kTwoLevelSplits > total4 / 16 ? kTwoLevelSplits : total4 / 16) : S;
+  if (!L->range && plan.counters > (int64_t)d->batch * d->num_kv_heads && engine == 0 &&
+      most_splits * total4 >= kSharedFoldElements && (int64_t)S * d->num_kv_heads * d->batch <= cus)
+    a.fold_polls = 32 + (int)((int64_t)plan.pages_per_split * d->page_size / 8);
   a.nw = L->range ? rs.nw : plan.waves_per_group;
   a.groups = 0;
   a.unit_extra = 0;

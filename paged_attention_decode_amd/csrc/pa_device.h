@@ -30,6 +30,15 @@ constexpr int kMinBlocks = 16;
 constexpr int kMinBlocksShort = 4;
 // Units with more splits than this merge in two levels (groups of 16).
 constexpr int kTwoLevelSplits = 48;
+// A unit's workgroups fold its splits together from this many (split, row, 4
+// columns) elements on (256 KB of partials), and up to kTwoLevelSplits splits
+// (or 64 of the largest partials, 16 rows of 256): they wait on one line, one
+// arrival after the other (us alone / shared: 2 x 16384 of 16/1 at 256, 64
+// splits, 25.0 / 19.4; 2 x 32768 at 128, 64 splits, 16.8 / 17.3; 1 x 65536,
+// 128 splits, 17.2 / 20.3).  With half the partials it gains nothing (8 x 8192
+// of 16/1 at 128, 14.8 / 15.5).
+constexpr int kSharedFoldElements = 16384;
+
 // LDS of one workgroup (wave merge + MFMA staging) is capped so that the
 // widest rows (head_dim 256, 16-row groups) still get 4 waves in a
 // workgroup that fits a CU's 160 KB: one 2-wave workgroup per split left
@@ -58,6 +67,7 @@ struct Phase1Args {
   int wl_key;      // key of the launch's plan, matched against the work list's header
   float scale_log2;
   float v_fix;     // fp8 caches: V's scale, applied to the output rows
+  int fold_polls;  // > 0: a unit's workgroups share the fold of its splits, each waiting at most this many polls
   const int32_t* bt;      // dense: block_table [B, max_pages]; CSR: indices
   const int32_t* sl;      // dense: seq_lens [B]
   const int32_t* indptr;  // CSR: [B + 1] offsets of each sequence's page ids in bt
@@ -229,6 +239,17 @@ struct MergeBatch {
     for (int j = 0; j < N; ++j)
       o[j] = load_device_f4(o_rsrc, ((uint32_t)((sp0 + j) * stride * gqa + row) * (uint32_t)d + col) * 4u);
   }
+  // Entries at or past `end`, inside the unit's region, load as zeros.
+  __device__ __forceinline__ void load_below(__amdgpu_buffer_rsrc_t o_rsrc, __amdgpu_buffer_rsrc_t ml_rsrc, int sp0,
+                                             int end, int gqa, int row, int col, int d) {
+    constexpr uint32_t kPast = 0x7ffffff0u;  // past any region
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      ml[j] = load_device_f2(ml_rsrc, sp0 + j < end ? (uint32_t)((sp0 + j) * gqa + row) * 8u : kPast);
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      o[j] = load_device_f4(o_rsrc, sp0 + j < end ? ((uint32_t)((sp0 + j) * gqa + row) * (uint32_t)d + col) * 4u : kPast);
+  }
   // Entries at or past `end` fold with m_s = -inf, i.e. weight 0 (their
   // loads read zeros: they lie past the unit's region): the fold has no
   // branch, so the compiler cannot sink a load into a conditional step and
@@ -272,6 +293,30 @@ __device__ __forceinline__ void merge_partials(__amdgpu_buffer_rsrc_t o_rsrc, __
   for (int sp0 = first; sp0 < end; sp0 += 16) {
     MergeBatch<16> p;
     p.load(o_rsrc, ml_rsrc, sp0, stride, gqa, row, col, d);
+    p.fold(sp0, end, m, l, acc);
+  }
+}
+
+// Folds (m_s, l_s, O_s) into (m, l, acc).
+__device__ __forceinline__ void fold_state(float ms, float ls, f4_t os, float& m, float& l, f4_t& acc) {
+  const float m_new = fmaxf(m, ms);
+  const float alpha = exp2_fast(m - m_new);  // 0 while m is -inf
+  const float beta = exp2_fast(ms - m_new);
+  l = l * alpha + ls * beta;
+  acc = acc * alpha + os * beta;
+  m = m_new;
+}
+
+// Folds entries [first, end) of one element in batches of 4, to a state of
+// its own.
+__device__ __forceinline__ void fold_run(__amdgpu_buffer_rsrc_t o_rsrc, __amdgpu_buffer_rsrc_t ml_rsrc, int first,
+                                         int end, int gqa, int row, int col, int d, float& m, float& l, f4_t& acc) {
+  m = kNegInf;
+  l = 0.f;
+  acc = (f4_t)0.f;
+  for (int sp0 = first; sp0 < end; sp0 += 4) {
+    MergeBatch<4> p;
+    p.load_below(o_rsrc, ml_rsrc, sp0, end, gqa, row, col, d);
     p.fold(sp0, end, m, l, acc);
   }
 }

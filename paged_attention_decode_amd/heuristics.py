@@ -38,6 +38,7 @@ OVERSUBSCRIBE_SPLITS = 4   # items per unit on an oversubscribed grid, at least,
 OVERSUBSCRIBE_GROUPS_PER_CU = 8  # and at least this many workgroups per CU
 PLAN_MAX_BATCH = 256       # largest batch the in-kernel planner handles
 TWO_LEVEL_SPLITS = 48      # units with more splits merge in two levels (groups of 16)
+SHARED_FOLD_ELEMENTS = 16384  # (split, row, 4 columns) elements from which a unit shares its fold
 RANGE_MAX_BATCH = 512      # largest batch a range launch takes
 RANGE_ROW_BYTES = 3 << 19  # fewest fp16 K/V bytes of a full table row in one head group
 RANGE_CALL_BYTES = 1 << 27  # and of all rows and groups
@@ -142,7 +143,10 @@ def plan_units(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, p
         s = num_splits
         pps = _cdiv(mp, s)
     else:
-        max_groups = num_cus // 2 if latency_bound else num_cus
+        fit = num_cus // units
+        shared_fold = (engine == 0 and fit <= TWO_LEVEL_SPLITS
+                       and fit * (num_q_heads // num_kv_heads) * (head_dim // 4) >= SHARED_FOLD_ELEMENTS)
+        max_groups = num_cus // 2 if latency_bound and not shared_fold else num_cus
         want = 1
         while want * 2 * units <= max_groups:
             want *= 2
