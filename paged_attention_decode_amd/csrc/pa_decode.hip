@@ -1806,14 +1806,26 @@ static int plan_key(const RangeArgs& a) {
   return (int)(h & 0x7fffffff);
 }
 
+// Bytes of a work list: header plus one record per workgroup (of either
+// kernel's grid), and of the per-unit grid of this plan.
+static_assert(kRlHeaderInts == kWlHeaderInts && kRlRecordInts == kWlRecordInts, "one size for both kernels' lists");
+static size_t worklist_bytes_of(int64_t groups) {
+  return sizeof(int32_t) * (size_t)(kWlHeaderInts + kWlRecordInts * groups);
+}
+static size_t worklist_bytes_for(const pad_decode_plan_t& plan, const pad_decode_dims* d) {
+  return worklist_bytes_of((int64_t)plan.num_splits * d->num_kv_heads * d->batch);
+}
+
 // Dense page table: bt = block_table, sl = seq_lens, indptr = lpl = NULL.
 // CSR: bt = indices, indptr / lpl given, sl unused (dims->max_pages is the
 // number of entries in indices).  io: also check q/k/v/out and the scratch
-// (a work-list plan reads only the index arrays).
+// (a work-list plan reads only the index arrays).  list_bytes: size of the
+// work list the launch reads or the plan writes, if there is one.
 static int setup_launch(const void* q, const void* k, const void* v, const int32_t* bt, const int32_t* sl,
                         const int32_t* indptr, const int32_t* lpl, void* out, void* ws, size_t ws_bytes,
                         int32_t* counters, int64_t num_counters, const pad_decode_dims* d, float scale,
-                        int num_splits, int engine, bool io, Launch* L, int kv_bytes = 2) {
+                        int num_splits, int engine, bool io, Launch* L, int kv_bytes = 2,
+                        size_t list_bytes = SIZE_MAX) {
   if (engine != 0 && engine != 1) return PAD_ERR_INVALID_SHAPE;
   // Page ids are bounds-checked against num_pages on the device (an id
   // outside [0, num_pages) reads page 0), so a launch that reads pages needs
@@ -1828,7 +1840,11 @@ static int setup_launch(const void* q, const void* k, const void* v, const int32
   st = plan_units(d, num_splits, cus, engine, csr, &plan, kv_bytes, &pps_full);
   if (st != PAD_OK) return st;
   const RangeShape rs = range_shape(d, num_splits, cus, engine, csr, kv_bytes);
-  L->range = rs.groups > 0 && (!io || (ws && ws_bytes >= rs.workspace_bytes && counters && num_counters >= rs.counters));
+  // The range kernel runs where its scratch and its list fit (an fp8 launch's
+  // own grid may have fewer workgroups than the range launch, and a list of
+  // that size stays good for it).
+  L->range = rs.groups > 0 && list_bytes >= worklist_bytes_of(rs.groups) &&
+             (!io || (ws && ws_bytes >= rs.workspace_bytes && counters && num_counters >= rs.counters));
   const int gqa = d->num_q_heads / d->num_kv_heads;
   if (engine == 1 && !valu_supported(d->head_dim, gqa)) return PAD_ERR_UNSUPPORTED_GQA;
   L->empty = d->batch == 0;
@@ -1955,12 +1971,6 @@ static int setup_launch(const void* q, const void* k, const void* v, const int32
   return PAD_OK;
 }
 
-// Bytes of the work list of this plan: header plus one record per workgroup.
-static size_t worklist_bytes_for(const pad_decode_plan_t& plan, const pad_decode_dims* d) {
-  const int64_t G = (int64_t)plan.num_splits * d->num_kv_heads * d->batch;
-  return sizeof(int32_t) * (size_t)(kWlHeaderInts + kWlRecordInts * G);
-}
-
 // A known format; bfloat16 and fp8 on the MFMA engine; fp8 with head_dim
 // 64/128/256 and finite positive scales (the scales are read for fp8 only).
 static bool kv_format_fp8(int f) {
@@ -2002,7 +2012,7 @@ static int launch_impl(const void* q, const void* k, const void* v, const int32_
   Launch L;
   const bool fp8 = kv_format_fp8(kv_format);
   st = setup_launch(q, k, v, bt, sl, indptr, lpl, out, ws, ws_bytes, counters, num_counters, d, scale,
-                    num_splits, engine, true, &L, fp8 ? 1 : 2);
+                    num_splits, engine, true, &L, fp8 ? 1 : 2, worklist ? worklist_bytes : SIZE_MAX);
   if (st != PAD_OK || L.empty) return st;
   if (fp8) {
     // The caches hold K / k_scale and V / v_scale: k_scale multiplies every
@@ -2060,7 +2070,7 @@ static int plan_worklist_impl(const int32_t* bt, const int32_t* sl, const int32_
                               void* stream, int kv_bytes = 2) {
   Launch L;
   int st = setup_launch(nullptr, nullptr, nullptr, bt, sl, indptr, lpl, nullptr, nullptr, 0, nullptr, 0, d, 1.0f,
-                        num_splits, 0, false, &L, kv_bytes);
+                        num_splits, 0, false, &L, kv_bytes, worklist_bytes);
   if (st != PAD_OK) return st;
   if (!worklist) return PAD_ERR_NULL_POINTER;
   if (worklist_bytes < worklist_bytes_for(L.plan, d)) return PAD_ERR_WORKSPACE;

@@ -11,6 +11,11 @@ namespace pad {
 // in up to 8 registers, and its work list two sequences per record.
 constexpr int kRangeMaxBatch = 512;
 
+// Work list of a range launch: as many int32 per record, and in the header, as
+// in the per-unit kernel's lists (pa_decode.hip checks both sizes at once).
+constexpr int kRlHeaderInts = 32;
+constexpr int kRlRecordInts = 32;
+
 // A range launch: Phase1Args with hkv counting head groups, and
 struct RangeArgs : Phase1Args {
   int groups;        // workgroups of the grid (G)

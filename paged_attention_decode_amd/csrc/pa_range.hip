@@ -714,8 +714,6 @@ __device__ __forceinline__ Piece piece_of(const Unit& u, int E, int T, int lo, i
 // unused, raw first page ids of the first segment's first 8 blocks (whole-page
 // blocks), then sequences 2g and 2g + 1 of the batch as {pages, tokens, CSR
 // row, owner of its zero rows or -1}}.
-constexpr int kRlHeaderInts = 32;
-constexpr int kRlRecordInts = 32;
 constexpr int kRlMagic = 0x574c4150;  // "PALW"
 
 __device__ __forceinline__ const int32_t* list_sequence(const RangeArgs& a, int b) {

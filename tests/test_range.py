@@ -141,6 +141,68 @@ def test_least_scratch_runs_the_per_unit_kernel():
         assert int(counters.abs().sum()) == 0
 
 
+# fp8 calls whose own grid has fewer workgroups than the range launch.
+SHORT_LISTS = [(129, 1, 8, 128, 16, 4096), (9, 8, 4, 128, 16, 4096)]  # batch, kv heads, group, head_dim, page size, table
+
+
+def _fp8_records(batch, hkv, group, d, ps, room):
+    return heuristics.plan_units(batch, hkv * group, hkv, d, ps, room // ps, kv_bytes=1).num_splits * batch * hkv
+
+
+@pytest.mark.parametrize("shape", SHORT_LISTS)
+def test_fp8_grids_smaller_than_the_range_launch(shape):
+    batch, hkv, group, d, ps, room = shape
+    groups, _, _ = heuristics.range_launch(batch, hkv * group, hkv, d, ps, room // ps, kv_bytes=1)
+    assert _fp8_records(*shape) < groups
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHORT_LISTS)
+def test_worklist_of_the_fp8_grids_size_is_not_overrun(shape):
+    """A list with room for the per-unit grid only is planned and run per unit; a shorter one is refused."""
+    batch, hkv, group, d, ps, room = shape
+    lib = _native.capi()
+    lens, q, k, v, bt, sl = _inputs(("ragged", batch, hkv, group, d, ps, room, "fp16", "e4m3"))
+    expected = decode_fp16_protocol(q.float(), k.float(), v.float(), bt, sl)
+    q, k, v, bt, sl = q.cuda(), k.cuda(), v.cuda(), bt.cuda(), sl.cuda()
+    out = torch.empty_like(q)
+    dm = _native.dims_for(q, k, v, bt, sl, out)
+    ws, n = ctypes.c_size_t(), ctypes.c_int64()
+    assert lib.pad_decode_workspace_bytes(ctypes.byref(dm), 0, 0, ctypes.byref(ws)) == 0
+    assert lib.pad_decode_counters_needed(ctypes.byref(dm), 0, 0, ctypes.byref(n)) == 0
+    workspace = torch.empty(ws.value, dtype=torch.uint8, device="cuda")
+    counters = torch.zeros(n.value, dtype=torch.int32, device="cuda")
+    full, least = ctypes.c_size_t(), 128 * (1 + _fp8_records(*shape))
+    assert lib.pad_decode_worklist_bytes(ctypes.byref(dm), 0, 0, 0, ctypes.byref(full)) == 0
+    assert least < full.value
+    worklist = torch.empty(full.value, dtype=torch.uint8, device="cuda")
+    c = _native.PadCall()
+    c.q, c.k_cache, c.v_cache, c.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
+    c.block_table, c.seq_lens = bt.data_ptr(), sl.data_ptr()
+    c.workspace, c.workspace_bytes = workspace.data_ptr(), ws.value
+    c.counters, c.num_counters = counters.data_ptr(), n.value
+    c.scale, c.kv_format, c.k_scale, c.v_scale = d ** -0.5, 1, 1.0, 1.0
+    c.worklist = worklist.data_ptr()
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def plan(nbytes):
+        return lib.pad_decode_plan_worklist_call(ctypes.byref(c), ctypes.byref(dm), worklist.data_ptr(), nbytes, stream)
+
+    for nbytes in (least, least + 128, full.value):
+        worklist.fill_(0x5A)
+        out.zero_()
+        assert plan(nbytes) == 0
+        c.worklist_bytes = nbytes
+        assert lib.pad_decode_launch_call(ctypes.byref(c), ctypes.byref(dm), stream) == 0
+        torch.cuda.synchronize()
+        assert bool((worklist[nbytes:] == 0x5A).all())
+        _check(out, expected, "fp16")
+        assert int(counters.abs().sum()) == 0
+    c.worklist_bytes = least - 1
+    assert plan(least - 1) == 7  # PAD_ERR_WORKSPACE
+    assert lib.pad_decode_launch_call(ctypes.byref(c), ctypes.byref(dm), stream) == 7
+
+
 def test_shapes_that_take_the_range_kernel():
     r = heuristics.range_launch
     assert r(256, 64, 8, 128, 16, 2048) == (256, 4, 4)
