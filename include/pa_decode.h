@@ -203,14 +203,14 @@ int pad_decode_least_scratch(const pad_decode_dims* dims, int num_splits,
  * harnesses that forbid allocation.  No counterpart in the reference.  The
  * split scratch is a static device
  * array of the library, one per GPU, of PAD_NOALLOC_WORKSPACE_BYTES bytes of
- * partials and PAD_NOALLOC_COUNTERS counters; a call whose plan
- * (pad_decode_workspace_bytes() / pad_decode_counters_needed()) needs more
- * returns PAD_ERR_SCRATCH_LIMIT without launching.  The first call on a
+ * partials and PAD_NOALLOC_COUNTERS counters; a call that cannot run with
+ * that (pad_decode_least_scratch()) returns PAD_ERR_SCRATCH_LIMIT without
+ * launching.  The first call on a
  * device looks up its copy's address and queues a small kernel that zeroes
  * the counters on `stream`.  Every call on one GPU shares that GPU's array:
  * calls that may overlap on one GPU (different streams, or graphs replayed
  * concurrently) race and must be serialised by the caller.  Same kernels,
- * plan and results as pad_decode_launch(). */
+ * plan and results as pad_decode_launch() with that much scratch. */
 int pad_decode_launch_noalloc(const void* q, const void* k_cache,
                               const void* v_cache, const int32_t* block_table,
                               const int32_t* seq_lens, void* out,

@@ -2137,8 +2137,10 @@ static int launch_noalloc(const void* q, const void* k, const void* v, const int
   int cus = 0;
   int st = device_cus(&cus);
   if (st != PAD_OK) return st;
+  // What the launch needs at least: one whose range launch does not fit the
+  // static scratch runs the per-unit kernel.
   pad_decode_plan_t plan;
-  st = plan_impl(d, num_splits, cus, 0, false, &plan);
+  st = plan_units(d, num_splits, cus, 0, false, &plan);
   if (st != PAD_OK) return st;
   if (plan.workspace_bytes > PAD_NOALLOC_WORKSPACE_BYTES || plan.counters > PAD_NOALLOC_COUNTERS)
     return PAD_ERR_SCRATCH_LIMIT;

@@ -203,6 +203,30 @@ def test_worklist_of_the_fp8_grids_size_is_not_overrun(shape):
     assert lib.pad_decode_launch_call(ctypes.byref(c), ctypes.byref(dm), stream) == 7
 
 
+@pytest.mark.gpu
+def test_noalloc_runs_per_unit_where_the_range_scratch_does_not_fit():
+    """65790 units: the range launch would count past the static counters, the per-unit kernel needs none."""
+    batch, heads, d, ps, width = 510, 129, 32, 16, 768
+    lib = _native.capi()
+    p = heuristics.plan(batch, heads, heads, d, ps, width)
+    assert p.counters > 65536 and heuristics.plan_units(batch, heads, heads, d, ps, width).single_pass
+    rng = random.Random(5)
+    lens = [rng.choice([0, 1, 15, 16, 17, 40]) for _ in range(batch)]
+    bt, num_pages = shuffled_table([16 * 8], ps, spare_pages=0, extra_cols=width - 8, seed=1)
+    bt = bt.expand(batch, width).contiguous()
+    k, v = make_cache(num_pages, ps, heads, d, seed=2)
+    q = torch.randn(batch, heads, d, generator=torch.Generator().manual_seed(3)).half()
+    k, v, sl = k.half(), v.half(), torch.tensor(lens, dtype=torch.int32)
+    expected = decode_fp16_protocol(q.float(), k.float(), v.float(), bt, sl)
+    q, k, v, bt, sl = q.cuda(), k.cuda(), v.cuda(), bt.cuda(), sl.cuda()
+    out = torch.full_like(q, float("nan"))
+    dm = _native.dims_for(q, k, v, bt, sl, out)
+    assert lib.pad_decode_launch_noalloc(q.data_ptr(), k.data_ptr(), v.data_ptr(), bt.data_ptr(), sl.data_ptr(),
+                                         out.data_ptr(), ctypes.byref(dm), ctypes.c_float(d ** -0.5), 0,
+                                         torch.cuda.current_stream().cuda_stream) == 0
+    _check(out, expected, "fp16")
+
+
 def test_shapes_that_take_the_range_kernel():
     r = heuristics.range_launch
     assert r(256, 64, 8, 128, 16, 2048) == (256, 4, 4)
