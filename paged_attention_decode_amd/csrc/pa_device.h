@@ -97,7 +97,11 @@ struct Phase1Args {
 __device__ __forceinline__ int page_of(const Phase1Args& a, int t) {
   return a.ps_shift >= 0 ? (t >> a.ps_shift) : t / a.ps;
 }
-__device__ __forceinline__ int pages_for(const Phase1Args& a, int n) { return page_of(a, n + a.ps - 1); }
+// (n + ps - 1 can pass 2^31 where a length lies far beyond its table: unsigned.)
+__device__ __forceinline__ int pages_for(const Phase1Args& a, int n) {
+  const uint32_t t = (uint32_t)n + (uint32_t)a.ps - 1u;
+  return (int)(a.ps_shift >= 0 ? t >> a.ps_shift : t / (uint32_t)a.ps);
+}
 // 16-token block -> page index (page_size a multiple of 16).
 __device__ __forceinline__ int block_page(const Phase1Args& a, int jb) {
   return a.ps_shift >= 4 ? (jb >> (a.ps_shift - 4)) : jb / (a.ps / 16);

@@ -227,6 +227,25 @@ def test_noalloc_runs_per_unit_where_the_range_scratch_does_not_fit():
     _check(out, expected, "fp16")
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("ps", [16, 12, 1])
+def test_lengths_far_past_the_table_are_clipped_to_it(ps):
+    """Lengths up to 2^31 - 1 name every page of their row, in the range kernel and in the per-unit kernel."""
+    import paged_attention_decode_amd as pad
+
+    batch, hkv, group, d, room = 40, 4, 4, 128, 2048
+    lens, q, k, v, bt, _ = _inputs(("ragged", batch, hkv, group, d, ps, room, "fp16", "fp16"))
+    cap = bt.shape[1] * ps
+    given = list(lens)
+    for b, n in ((2, 2**31 - 1), (5, 2**31 - ps), (9, 2**31 - ps - 1), (30, cap + 1)):
+        lens[b], given[b] = cap, n
+    expected = decode_fp16_protocol(q.float(), k.float(), v.float(), bt, torch.tensor(lens, dtype=torch.int32))
+    q, k, v, bt, sl = q.cuda(), k.cuda(), v.cuda(), bt.cuda(), torch.tensor(given, dtype=torch.int32).cuda()
+    assert heuristics.range_launch(batch, hkv * group, hkv, d, ps, bt.shape[1]) is not None
+    for splits in (None, 3):  # 3: the per-unit kernel
+        _check(pad.paged_attention_decode_ex(q, k, v, bt, sl, num_splits=splits), expected, "fp16")
+
+
 def test_shapes_that_take_the_range_kernel():
     r = heuristics.range_launch
     assert r(256, 64, 8, 128, 16, 2048) == (256, 4, 4)
