@@ -624,7 +624,12 @@ struct Sequences {
 // counts E = unit_extra positions at its front, T = ceil(P / G), at least
 // min_chunk.  All the same page count: the units are cut alike, into as many
 // pieces as ranges are left for each (E fills a unit up to whole ranges), or
-// each range takes as many whole units.
+// each range takes as many whole units - unless that leaves so much of the
+// grid idle that the ranges are more than 1.6 times as long.  us cut alike /
+// into equal ranges, by that ratio: 33 x 4096 of 32/8 heads (1.26) 88 / 92, 43
+// (1.45) 113.8 / 114.9, 150 of 8/1 (1.58) 54.1 / 57.1, 72 of 32/8 (1.74) 208 /
+// 194, 65 (1.92) 189 / 170, 129 (1.94) 367 / 325; 65 x 8192 at head_dim 64
+// (1.92) 219 / 166.
 // Empty sequences lie between units without a page; the workgroup whose range
 // holds that position (the last range at the end) writes their zero rows:
 // on_empty(b, owner) is called by the lane of every empty sequence b.  NK
@@ -649,19 +654,21 @@ __device__ __forceinline__ RangePlan plan_ranges(const RangeArgs& a, int g, int 
   used = wave_sum_i32(used) * a.hkv;
   most = wave_max_i32(most);
   p.E = a.unit_extra;
+  p.P = tot * a.hkv + used * p.E;
+  p.T = max((p.P + a.groups - 1) / a.groups, max(a.min_chunk, 1));
   if (__builtin_amdgcn_ballot_w64(least < most) == 0 && used > 0) {
-    const int pages = most;
+    int T, E = 0;
     if (used <= a.groups) {
-      p.T = max((pages + a.groups / used - 1) / (a.groups / used), a.min_chunk);
-      p.E = (pages + p.T - 1) / p.T * p.T - pages;
+      T = max((most + a.groups / used - 1) / (a.groups / used), a.min_chunk);
+      E = (most + T - 1) / T * T - most;
     } else {
-      p.T = (used + a.groups - 1) / a.groups * pages;
-      p.E = 0;
+      T = (used + a.groups - 1) / a.groups * most;
     }
-    p.P = used * (pages + p.E);
-  } else {
-    p.P = tot * a.hkv + used * p.E;
-    p.T = max((p.P + a.groups - 1) / a.groups, max(a.min_chunk, 1));
+    if (5 * (int64_t)T <= 8 * (int64_t)p.T) {
+      p.T = T;
+      p.E = E;
+      p.P = used * (most + E);
+    }
   }
   const int lo = g * p.T;
   p.first = Unit{};

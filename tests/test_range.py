@@ -246,6 +246,36 @@ def test_lengths_far_past_the_table_are_clipped_to_it(ps):
         _check(pad.paged_attention_decode_ex(q, k, v, bt, sl, num_splits=splits), expected, "fp16")
 
 
+# Equal lengths whose units do not divide the grid: cut alike, or in whole units, up to half of it would be idle.
+EQUAL_SHAPES = [(65, 8, 1024), (72, 8, 1024), (129, 8, 768), (140, 8, 768), (257, 1, 3072), (64, 8, 1024), (33, 8, 1024),
+                (200, 4, 1024)]  # batch, kv heads, tokens; the last three are cut alike
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", EQUAL_SHAPES, ids=lambda s: "-".join(map(str, s)))
+def test_equal_lengths_keep_the_grid_busy(shape):
+    """Read from the work list: no range is more than 1.6 times as long as an equal share of the positions."""
+    import paged_attention_decode_amd as pad
+
+    batch, hkv, tokens = shape
+    group, d, ps = 2, 128, 16
+    pages = tokens // ps
+    groups, heads, _ = heuristics.range_launch(batch, hkv * group, hkv, d, ps, pages)
+    lens, q, k, v, bt, sl = _inputs(("equal", batch, hkv, group, d, ps, tokens, "fp16", "fp16"))
+    expected = decode_fp16_protocol(q.float(), k.float(), v.float(), bt, sl)
+    q, k, v, bt, sl = q.cuda(), k.cuda(), v.cuda(), bt.cuda(), sl.cuda()
+    w = pad.BatchDecodeWrapper()
+    w.plan_block_table(bt, sl, hkv * group, hkv, d, ps)
+    records = w._plan[2].view(torch.int32)[32:32 + 32 * groups].view(groups, 32).cpu()
+    T, P = int(records[0, 11]), int(records[0, 12])
+    units = batch * hkv // heads
+    extra = -(-160 * 1024 // (ps * d * 4 * heads))  # positions of a unit beyond its pages
+    assert int((records[:, 8] != 0).sum()) == -(-P // T) <= groups
+    assert 5 * T <= 8 * -(-units * (pages + extra) // groups)
+    _check(w.run(q, (k, v)), expected, "fp16")
+    _check(pad.paged_attention_decode(q, k, v, bt, sl), expected, "fp16")
+
+
 def test_shapes_that_take_the_range_kernel():
     r = heuristics.range_launch
     assert r(256, 64, 8, 128, 16, 2048) == (256, 4, 4)
