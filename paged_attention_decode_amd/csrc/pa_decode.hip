@@ -1650,8 +1650,23 @@ static RangeShape range_shape(const pad_decode_dims* d, int num_splits, int num_
   if (num_cus <= 0) num_cus = 256;
   const int64_t units = (int64_t)d->batch * d->num_kv_heads;
   if (num_splits != 0 || engine != 0 || d->batch <= 0 || d->batch > kRangeMaxBatch || d->num_kv_heads == 2) return r;
-  if (units * 4 <= num_cus || units * 2 == num_cus || latency_bound_shape(d, num_cus, csr)) return r;
   r.nh_shift = d->num_kv_heads % 4 == 0 ? 2 : (d->num_kv_heads % 2 == 0 ? 1 : 0);
+  // Rows of at most 128 bytes: 8 waves keep as many bytes in flight as 4 of
+  // wider rows (fp8, 64 x [1, 8192]: 93.3 us with 8, 93.8 with 4; head_dim 64,
+  // 24 x [1, 4096]: 22.5 and 23.1 us).
+  r.nw = d->head_dim * kv_bytes <= 128 ? kMaxWaves : kMaxWaves / 2;
+  // Units: above a quarter of one per CU, as the oversubscribed grid, and not
+  // at one per two CUs, whose splits the per-unit grid deals evenly.  Groups of
+  // four heads need more, as a workgroup's waves then stream a head each (one
+  // wave, or two of fp8 rows) and a call of few units waits for that: speed
+  // against the per-unit kernel at 72 / 96 / 136 units, 9 / 12 / 17 x [1, n]
+  // of 64/8 heads: n = 3632 0.68 / 0.76 (3456) / 0.95 (3872), full tables of
+  // 4096 0.82 / 0.89 / 1.22; 17 and 24 x [1, 1920] of 16/4 at 256 0.82, 0.88;
+  // fp8, 9 and 12 x [1, 4096] of 32/8 0.91, 1.28, full 0.93, 1.03.  One and two
+  // heads per workgroup gain from 70 units on (70 x [1, 4736] of 8/1 1.11, 12 x
+  // [1, 4608] of 24/6 1.05), and so does head_dim 64 (9 x [1, 7264] 1.32).
+  if (units * 4 <= num_cus || units * 2 == num_cus || latency_bound_shape(d, num_cus, csr)) return r;
+  if (r.nh_shift == 2 && (r.nw == kMaxWaves / 2 ? units * 2 < num_cus : kv_bytes == 1 && units * 3 <= num_cus)) return r;
   const int64_t page_bytes = ((int64_t)d->page_size * d->head_dim * kv_bytes * 2) << r.nh_shift;
   const int64_t row_bytes = plan_pages_per_seq(d, csr) * (((int64_t)d->page_size * d->head_dim * 4) << r.nh_shift);
   if (row_bytes < kRangeRowBytes || (units >> r.nh_shift) * row_bytes < kRangeCallBytes) return r;
@@ -1664,10 +1679,6 @@ static RangeShape range_shape(const pad_decode_dims* d, int num_splits, int num_
   const int groups = (int)(records < num_cus ? records : num_cus);
   if (d->batch > 2 * groups) return r;
   r.groups = groups;
-  // Rows of at most 128 bytes: 8 waves keep as many bytes in flight as 4 of
-  // wider rows (fp8, 64 x [1, 8192]: 93.3 us with 8, 93.8 with 4; head_dim 64,
-  // 24 x [1, 4096]: 22.5 and 23.1 us).
-  r.nw = d->head_dim * kv_bytes <= 128 ? kMaxWaves : kMaxWaves / 2;
   r.unit_extra = ceil_div(kRangeUnitBytes, page_bytes);
   r.min_chunk = ceil_div(kRangeMinBytes, page_bytes);
   r.workspace_bytes = range_layout(d, r, nullptr, nullptr, nullptr);
@@ -1675,18 +1686,20 @@ static RangeShape range_shape(const pad_decode_dims* d, int num_splits, int num_
   return r;
 }
 
-// The plan of a launch, and of its range launch if the shape takes one
-// (range, may be null).  The scratch covers both: a launch with less than the
-// range kernel needs runs the per-unit kernel.
+// What pad_decode_plan() reports: the per-unit plan, with scratch for the range
+// launch too if the shape takes one (a launch with less runs the per-unit
+// kernel).  It sizes the scratch of 16-bit and fp8 launches: an fp8 launch may
+// take the range kernel where a 16-bit one does not.
 static int plan_impl(const pad_decode_dims* d, int num_splits, int num_cus, int engine, bool csr,
-                     pad_decode_plan_t* p, int kv_bytes = 2, int* pps_full = nullptr, RangeShape* range = nullptr) {
-  const int st = plan_units(d, num_splits, num_cus, engine, csr, p, kv_bytes, pps_full);
+                     pad_decode_plan_t* p) {
+  const int st = plan_units(d, num_splits, num_cus, engine, csr, p);
   if (st != PAD_OK) return st;
-  const RangeShape r = range_shape(d, num_splits, num_cus, engine, csr, kv_bytes);
-  if (range) *range = r;
-  if (r.groups > 0) {
+  const bool fp8_dim = d->head_dim == 64 || d->head_dim == 128 || d->head_dim == 256;
+  for (int kv_bytes = 2; kv_bytes >= (fp8_dim ? 1 : 2); --kv_bytes) {
+    const RangeShape r = range_shape(d, num_splits, num_cus, engine, csr, kv_bytes);
+    if (r.groups == 0) continue;
+    if (kv_bytes == 2) p->waves_per_group = r.nw;
     p->single_pass = 0;
-    p->waves_per_group = r.nw;
     if (p->workspace_bytes < r.workspace_bytes) p->workspace_bytes = r.workspace_bytes;
     if (p->counters < r.counters) p->counters = r.counters;
   }

@@ -89,16 +89,20 @@ def plan(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, page_si
     unit per CU up only: never more scratch), 8-wave workgroups for its 128-byte rows at head_dim 128."""
     p = plan_units(batch, num_q_heads, num_kv_heads, head_dim, page_size, max_pages, num_splits, num_cus, engine,
                    csr, kv_bytes)
-    r = None
-    if num_splits == 0 and engine == 0:
-        r = range_launch(batch, num_q_heads, num_kv_heads, head_dim, page_size, max_pages, num_cus, csr, kv_bytes)
-    if r is None:
+    if num_splits != 0 or engine != 0:
         return p
-    groups, heads, waves = r
-    rows = 2 * groups * heads * (num_q_heads // num_kv_heads)
-    return Plan(p.num_splits, p.pages_per_split, waves, False,
-                max(p.workspace_bytes, 256 + rows * head_dim * 4 + rows * 8),
-                max(p.counters, batch * num_kv_heads // heads + 2 * groups))
+    # The 16-bit plan sizes the scratch of an fp8 launch too.
+    widths = (2, 1) if kv_bytes == 2 and head_dim in (64, 128, 256) else (kv_bytes,)
+    for es in widths:
+        r = range_launch(batch, num_q_heads, num_kv_heads, head_dim, page_size, max_pages, num_cus, csr, es)
+        if r is None:
+            continue
+        groups, heads, waves = r
+        rows = 2 * groups * heads * (num_q_heads // num_kv_heads)
+        p = Plan(p.num_splits, p.pages_per_split, waves if es == kv_bytes else p.waves_per_group, False,
+                 max(p.workspace_bytes, 256 + rows * head_dim * 4 + rows * 8),
+                 max(p.counters, batch * num_kv_heads // heads + 2 * groups))
+    return p
 
 
 def range_launch(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, page_size: int, max_pages: int,
@@ -106,7 +110,9 @@ def range_launch(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int,
     """(workgroups, kv heads per workgroup, waves) of a heuristic launch that takes the range kernel, or None.
 
     Bandwidth-bound shapes with units as the oversubscribed grid takes them
-    and batch <= RANGE_MAX_BATCH, except two kv heads and short table rows."""
+    (groups of four heads: above one unit per two CUs, per three with fp8 rows
+    of 128 bytes) and batch <= RANGE_MAX_BATCH, except two kv heads and short
+    table rows."""
     if num_cus <= 0:
         num_cus = 256
     units = batch * num_kv_heads
@@ -117,6 +123,9 @@ def range_launch(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int,
     if units * 4 <= num_cus or units * 2 == num_cus or latency_bound:
         return None
     heads = 4 if num_kv_heads % 4 == 0 else 2 if num_kv_heads % 2 == 0 else 1
+    waves = MAX_WAVES if head_dim * kv_bytes <= 128 else MAX_WAVES // 2
+    if heads == 4 and (units * 2 < num_cus if waves < MAX_WAVES else kv_bytes == 1 and units * 3 <= num_cus):
+        return None
     row_bytes = mp * page_size * head_dim * 4 * heads
     if row_bytes < RANGE_ROW_BYTES or units // heads * row_bytes < RANGE_CALL_BYTES:
         return None
@@ -126,7 +135,7 @@ def range_launch(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int,
     groups = min(units * p.num_splits, num_cus)
     if batch > 2 * groups:
         return None
-    return groups, heads, MAX_WAVES if head_dim * kv_bytes <= 128 else MAX_WAVES // 2
+    return groups, heads, waves
 
 
 def plan_units(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, page_size: int, max_pages: int,

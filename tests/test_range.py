@@ -142,7 +142,7 @@ def test_least_scratch_runs_the_per_unit_kernel():
 
 
 # fp8 calls whose own grid has fewer workgroups than the range launch.
-SHORT_LISTS = [(129, 1, 8, 128, 16, 4096), (9, 8, 4, 128, 16, 4096)]  # batch, kv heads, group, head_dim, page size, table
+SHORT_LISTS = [(129, 1, 8, 128, 16, 4096), (12, 8, 4, 128, 16, 4096)]  # batch, kv heads, group, head_dim, page size, table
 
 
 def _fp8_records(batch, hkv, group, d, ps, room):
@@ -274,6 +274,20 @@ def test_equal_lengths_keep_the_grid_busy(shape):
     assert 5 * T <= 8 * -(-units * (pages + extra) // groups)
     _check(w.run(q, (k, v)), expected, "fp16")
     _check(pad.paged_attention_decode(q, k, v, bt, sl), expected, "fp16")
+
+
+def test_few_units_of_four_heads_stay_per_unit():
+    r = heuristics.range_launch
+    assert r(10, 64, 8, 128, 16, 208) is None and r(11, 64, 8, 128, 16, 202) is None  # 0.7 of the per-unit kernel's speed
+    assert r(9, 32, 8, 128, 16, 4096) is None and r(24, 16, 4, 256, 16, 256) is None
+    assert r(16, 32, 8, 128, 16, 512) is None and r(17, 32, 8, 128, 16, 512) == (256, 4, 4)
+    assert r(9, 32, 8, 128, 16, 512, kv_bytes=1) is None and r(12, 32, 8, 128, 16, 256, kv_bytes=1) is not None
+    assert r(9, 32, 8, 64, 16, 512) is not None  # 128-byte rows
+    assert r(12, 24, 6, 128, 16, 288) is not None and r(70, 8, 1, 128, 16, 296) is not None  # one and two heads
+    # the fp8 launch's scratch is in the 16-bit plan that sizes it
+    for group in (1, 4, 16):
+        plan = heuristics.plan(12, 8 * group, 8, 128, 16, 256)
+        assert plan.workspace_bytes >= 256 + 2 * 256 * 4 * group * (128 * 4 + 8) and plan.counters >= 24 + 2 * 256
 
 
 def test_shapes_that_take_the_range_kernel():
