@@ -127,13 +127,17 @@ typedef struct pad_decode_dims {
   int64_t out_stride[3];
 } pad_decode_dims;
 
-/* Work decomposition chosen for a call: the kernels walk
- * pages_per_split pages of one sequence per workgroup. */
+/* Work decomposition chosen for a call: the per-unit kernel walks
+ * pages_per_split pages of one sequence per workgroup.  A call of many units
+ * may run the range kernel instead (one workgroup per CU over equal page
+ * ranges): then the scratch below covers both kernels, and the other fields
+ * are still the per-unit kernel's, which runs with less scratch
+ * (pad_decode_least_scratch()). */
 typedef struct pad_decode_plan_t {
   int32_t num_splits;       /* splits per (sequence, kv head)              */
   int32_t pages_per_split;
   int32_t waves_per_group;  /* 64-lane waves per phase-1 workgroup         */
-  int32_t single_pass;      /* 1: one split per sequence, no partials      */
+  int32_t single_pass;      /* 1: the call takes no scratch                */
   int32_t engine;           /* 0 = MFMA tiles, 1 = VALU/DPP dot products   */
   int32_t reserved;
   size_t workspace_bytes;   /* fp32 partials; 0 if single_pass             */

@@ -1698,7 +1698,6 @@ static int plan_impl(const pad_decode_dims* d, int num_splits, int num_cus, int 
   for (int kv_bytes = 2; kv_bytes >= (fp8_dim ? 1 : 2); --kv_bytes) {
     const RangeShape r = range_shape(d, num_splits, num_cus, engine, csr, kv_bytes);
     if (r.groups == 0) continue;
-    if (kv_bytes == 2) p->waves_per_group = r.nw;
     p->single_pass = 0;
     if (p->workspace_bytes < r.workspace_bytes) p->workspace_bytes = r.workspace_bytes;
     if (p->counters < r.counters) p->counters = r.counters;

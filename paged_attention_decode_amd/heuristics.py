@@ -80,9 +80,9 @@ def plan(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, page_si
          num_splits: int = 0, num_cus: int = 256, engine: int = 0, csr: bool = False, kv_bytes: int = 2) -> Plan:
     """Same result as ``pad_decode_plan`` (``pad_decode_plan_csr`` with ``csr``) for valid arguments.
 
-    Where the launch takes the range kernel (``range_launch``), its waves, and
-    scratch for both it and the per-unit kernel, which a launch with less
-    scratch runs.
+    The per-unit kernel's splits and waves; where the launch takes the range
+    kernel (``range_launch`` has its grid), scratch for both, as a launch with
+    less runs the per-unit kernel.
 
     ``kv_bytes=1`` gives the plan of an fp8-cache launch (pad_decode_launch_kv8): the same splits and
     scratch except where the fp16 plan is an oversubscribed grid (fp8 takes the 4-item grid from one
@@ -97,9 +97,9 @@ def plan(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, page_si
         r = range_launch(batch, num_q_heads, num_kv_heads, head_dim, page_size, max_pages, num_cus, csr, es)
         if r is None:
             continue
-        groups, heads, waves = r
+        groups, heads, _ = r
         rows = 2 * groups * heads * (num_q_heads // num_kv_heads)
-        p = Plan(p.num_splits, p.pages_per_split, waves if es == kv_bytes else p.waves_per_group, False,
+        p = Plan(p.num_splits, p.pages_per_split, p.waves_per_group, False,
                  max(p.workspace_bytes, 256 + rows * head_dim * 4 + rows * 8),
                  max(p.counters, batch * num_kv_heads // heads + 2 * groups))
     return p

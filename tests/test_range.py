@@ -276,6 +276,27 @@ def test_equal_lengths_keep_the_grid_busy(shape):
     _check(pad.paged_attention_decode(q, k, v, bt, sl), expected, "fp16")
 
 
+def test_plans_describe_one_kernel():
+    """Splits, pages and waves of a plan are the per-unit kernel's; its scratch covers the range kernel too."""
+    lib = _native.capi()
+    taken = 0
+    for batch, hq, hkv, d, ps, pages in ((64, 32, 8, 128, 16, 512), (70, 32, 8, 64, 16, 512), (300, 8, 1, 128, 16, 256),
+                                         (33, 64, 4, 256, 16, 64), (100, 24, 6, 96, 16, 400), (8, 32, 8, 128, 16, 512)):
+        u = heuristics.plan_units(batch, hq, hkv, d, ps, pages)
+        m = heuristics.plan(batch, hq, hkv, d, ps, pages)
+        r = heuristics.range_launch(batch, hq, hkv, d, ps, pages)
+        taken += r is not None and r[2] != u.waves_per_group
+        q, k = torch.empty(batch, hq, d, dtype=torch.float16), torch.empty(1, ps, hkv, d, dtype=torch.float16)
+        index = torch.zeros(batch, pages, dtype=torch.int32)
+        p = _native.PadPlan()
+        dm = _native.dims_for(q, k, k, index, index[:, 0], q)
+        assert lib.pad_decode_plan(ctypes.byref(dm), 0, 256, ctypes.byref(p)) == 0
+        assert (p.num_splits, p.pages_per_split, p.waves_per_group) == (
+            u.num_splits, u.pages_per_split, u.waves_per_group) == (m.num_splits, m.pages_per_split, m.waves_per_group)
+        assert (bool(p.single_pass), p.workspace_bytes, p.counters) == (m.single_pass, m.workspace_bytes, m.counters)
+    assert taken >= 1
+
+
 def test_few_units_of_four_heads_stay_per_unit():
     r = heuristics.range_launch
     assert r(10, 64, 8, 128, 16, 208) is None and r(11, 64, 8, 128, 16, 202) is None  # 0.7 of the per-unit kernel's speed
