@@ -53,6 +53,11 @@ int pad_timeline_read(void* host, size_t bytes);
 /* Zero the stamp buffer and restart the launch count at 0; synchronous. */
 int pad_timeline_reset(void);
 
+/* Bound of the shared fold's wait in this library's next launches, in polls
+ * (0: the product's).  With 1, a unit's early workgroups give up, and its
+ * last arrival folds the unit. */
+int pad_timeline_set_fold_polls(int polls);
+
 #ifdef __cplusplus
 }  /* extern "C" */
 #endif

@@ -198,6 +198,7 @@ TIMELINE_PATH = os.path.join(_PKG_DIR, "libpa_decode_tl.so")
 TIMELINE_SIGNATURES = {
     "pad_timeline_read": ([_VP, ctypes.c_size_t], ctypes.c_int),
     "pad_timeline_reset": ([], ctypes.c_int),
+    "pad_timeline_set_fold_polls": ([ctypes.c_int], ctypes.c_int),
 }
 # include/pa_decode_timeline.h
 TL_LAUNCHES, TL_MAX_GROUPS, TL_SLOTS = 4, 16384, 8

@@ -64,6 +64,7 @@ namespace pad {
 // Slot meanings are the PAD_TL_* constants of pa_decode_timeline.h.
 __device__ unsigned long long tl_buf[PAD_TL_LAUNCHES * PAD_TL_MAX_GROUPS * PAD_TL_SLOTS];
 static int tl_launches = 0;
+static int tl_fold_polls = 0;  // pad_timeline_set_fold_polls()
 #define PAD_TL_AT(lin, slot, value)                                                                      \
   do {                                                                                                   \
     if (threadIdx.x == 0 && (lin) < PAD_TL_MAX_GROUPS)                                                   \
@@ -1219,11 +1220,11 @@ void pad_phase1_kernel(const Phase1Args a) {
             if (first < end) {
               float mr = kNegInf, lr = 0.f;
               f4_t ar = (f4_t)0.f;
-              p[i].fold(first, end, mr, lr, ar);
+              p[i].fold_states(first, end, mr, lr, ar);
               for (int sp0 = first + 4; sp0 < end; sp0 += 4) {
                 MergeBatch<4> q;
                 q.load_below(o_rsrc, ml_rsrc, sp0, end, gqa, row, col, D);
-                q.fold(sp0, end, mr, lr, ar);
+                q.fold_states(sp0, end, mr, lr, ar);
               }
               fold_state(mr, lr, ar, m, l, acc);
             }
@@ -1957,6 +1958,9 @@ static int setup_launch(const void* q, const void* k, const void* v, const int32
   if (!L->range && plan.counters > (int64_t)d->batch * d->num_kv_heads && engine == 0 &&
       most_splits * total4 >= kSharedFoldElements && (int64_t)S * d->num_kv_heads * d->batch <= cus)
     a.fold_polls = 32 + (int)((int64_t)plan.pages_per_split * d->page_size / 8);
+#ifdef PAD_TIMELINE
+  if (a.fold_polls > 0 && tl_fold_polls > 0) a.fold_polls = tl_fold_polls;
+#endif
   a.nw = L->range ? rs.nw : plan.waves_per_group;
   a.groups = 0;
   a.unit_extra = 0;
@@ -2376,6 +2380,11 @@ int pad_timeline_reset(void) {
   if (hipMemset(p, 0, sizeof(pad::tl_buf)) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
     return PAD_ERR_DEVICE;
   pad::tl_launches = 0;
+  return PAD_OK;
+}
+
+int pad_timeline_set_fold_polls(int polls) {
+  pad::tl_fold_polls = polls > 0 ? polls : 0;
   return PAD_OK;
 }
 #endif

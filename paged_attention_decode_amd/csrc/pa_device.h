@@ -222,6 +222,20 @@ __device__ __forceinline__ float2 load_device_f2(__amdgpu_buffer_rsrc_t r, uint3
   return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kCachePolicyDevice));
 }
 
+// Folds (m_s, l_s, O_s) into (m, l, acc), with its rounding spelled out: of a
+// sum of two products the compiler may fuse either one, and not the same one
+// wherever it compiles the fold, but a unit folded by all its workgroups and
+// one folded by its last arrival have to give the same bits.
+__device__ __forceinline__ void fold_state(float ms, float ls, f4_t os, float& m, float& l, f4_t& acc) {
+  const float m_new = fmaxf(m, ms);
+  const float alpha = exp2_fast(m - m_new);  // 0 while m is -inf
+  const float beta = exp2_fast(ms - m_new);
+  l = __builtin_fmaf(l, alpha, ls * beta);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(acc[i], alpha, os[i] * beta);
+  m = m_new;
+}
+
 // N consecutive splits' partials of one (row, 4 columns) element, loaded
 // with device-scope loads (the (m, l) pairs first, in split order, then the
 // O vectors) and folded in split order:
@@ -272,6 +286,11 @@ struct MergeBatch {
       m = m_new;
     }
   }
+  // The same, one fold_state() after the other.
+  __device__ __forceinline__ void fold_states(int sp0, int end, float& m, float& l, f4_t& acc) const {
+#pragma unroll
+    for (int j = 0; j < N; ++j) fold_state(sp0 + j < end ? ml[j].x : kNegInf, ml[j].y, o[j], m, l, acc);
+  }
 };
 
 // Folds entries [first, first + count) of one element (entry i in split
@@ -301,16 +320,6 @@ __device__ __forceinline__ void merge_partials(__amdgpu_buffer_rsrc_t o_rsrc, __
   }
 }
 
-// Folds (m_s, l_s, O_s) into (m, l, acc).
-__device__ __forceinline__ void fold_state(float ms, float ls, f4_t os, float& m, float& l, f4_t& acc) {
-  const float m_new = fmaxf(m, ms);
-  const float alpha = exp2_fast(m - m_new);  // 0 while m is -inf
-  const float beta = exp2_fast(ms - m_new);
-  l = l * alpha + ls * beta;
-  acc = acc * alpha + os * beta;
-  m = m_new;
-}
-
 // Folds entries [first, end) of one element in batches of 4, to a state of
 // its own.
 __device__ __forceinline__ void fold_run(__amdgpu_buffer_rsrc_t o_rsrc, __amdgpu_buffer_rsrc_t ml_rsrc, int first,
@@ -321,7 +330,7 @@ __device__ __forceinline__ void fold_run(__amdgpu_buffer_rsrc_t o_rsrc, __amdgpu
   for (int sp0 = first; sp0 < end; sp0 += 4) {
     MergeBatch<4> p;
     p.load_below(o_rsrc, ml_rsrc, sp0, end, gqa, row, col, d);
-    p.fold(sp0, end, m, l, acc);
+    p.fold_states(sp0, end, m, l, acc);
   }
 }
 

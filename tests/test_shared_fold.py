@@ -9,11 +9,14 @@ workgroups may give up waiting) write the bits of a launch alone.
 
 from __future__ import annotations
 
+import ctypes
+
+import numpy as np
 import pytest
 import torch
 
 from oracle.reference import decode_fp16_protocol
-from paged_attention_decode_amd import heuristics
+from paged_attention_decode_amd import _native, heuristics
 from tests.helpers import make_cache, shuffled_table
 
 DTYPES = {"fp16": torch.float16, "bf16": torch.bfloat16, "e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}
@@ -60,6 +63,61 @@ def test_shared_fold_against_oracle(case):
                 outs.append(decode(q, k, v, bt, sl))
     torch.cuda.synchronize()
     assert all(torch.equal(out, o) for o in outs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [CASES[i] for i in (0, 1, 3, 5)], ids=lambda c: f"b{len(c[0])}-{'-'.join(map(str, c[1:]))}")
+def test_workgroups_that_give_up_leave_the_same_bits(case):
+    """In the measurement library with one poll: a unit's early workgroups give up, and its last arrival folds it."""
+    import paged_attention_decode_amd as pad
+
+    lens, hkv, group, d, ps, qt, kvt = case
+    bt, num_pages = shuffled_table(lens, ps, spare_pages=2, extra_cols=0, seed=d)
+    k, v = make_cache(num_pages, ps, hkv, d, seed=len(lens))
+    q = torch.randn(len(lens), hkv * group, d, generator=torch.Generator().manual_seed(ps)).to(DTYPES[qt]).cuda()
+    k, v, bt = k.to(DTYPES[kvt]).cuda(), v.to(DTYPES[kvt]).cuda(), bt.cuda()
+    sl = torch.tensor(lens, dtype=torch.int32).cuda()
+    expected = pad.paged_attention_decode_ex(q, k, v, bt, sl)
+    lib = _native.timeline()
+    out = torch.empty_like(q)
+    dm = _native.dims_for(q, k, v, bt, sl, out)
+    ws, n = ctypes.c_size_t(), ctypes.c_int64()
+    assert lib.pad_decode_workspace_bytes(ctypes.byref(dm), 0, 0, ctypes.byref(ws)) == 0
+    assert lib.pad_decode_counters_needed(ctypes.byref(dm), 0, 0, ctypes.byref(n)) == 0
+    workspace = torch.empty(ws.value, dtype=torch.uint8, device="cuda")
+    counters = torch.zeros(n.value, dtype=torch.int32, device="cuda")
+    c = _native.PadCall()
+    c.q, c.k_cache, c.v_cache, c.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
+    c.block_table, c.seq_lens = bt.data_ptr(), sl.data_ptr()
+    c.workspace, c.workspace_bytes = workspace.data_ptr(), ws.value
+    c.counters, c.num_counters = counters.data_ptr(), n.value
+    c.scale, c.k_scale, c.v_scale, c.kv_format = d ** -0.5, 1.0, 1.0, 3 if qt == "bf16" else 0
+    shape = (_native.TL_LAUNCHES, _native.TL_MAX_GROUPS, _native.TL_SLOTS)
+    buf = np.zeros(shape, dtype=np.uint64)
+
+    def run(polls):
+        out.zero_()
+        assert lib.pad_timeline_reset() == 0 and lib.pad_timeline_set_fold_polls(polls) == 0
+        try:
+            st = lib.pad_decode_launch_call(ctypes.byref(c), ctypes.byref(dm), torch.cuda.current_stream().cuda_stream)
+        finally:
+            lib.pad_timeline_set_fold_polls(0)
+        assert st == 0
+        torch.cuda.synchronize()
+        assert torch.equal(out, expected)
+        assert int(counters.abs().sum()) == 0
+        assert lib.pad_timeline_read(buf.ctypes.data, buf.nbytes) == 0
+        rows = buf[0].astype(np.int64)
+        flags = rows[:, _native.TL_INFO] >> 40 & 0xFF
+        arrived = rows[:, _native.TL_ARRIVED] != 0
+        folded = (flags & _native.TL_F_MERGER) != 0
+        return int((arrived & folded).sum()), int((arrived & ~folded).sum())
+
+    for _ in range(3):
+        folded, gave_up = run(1)
+        assert folded > 0 and gave_up > 0, (folded, gave_up)
+    folded, gave_up = run(0)
+    assert folded > gave_up, (folded, gave_up)
 
 
 def test_split_counts_of_shared_folds():
