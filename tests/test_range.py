@@ -276,6 +276,233 @@ def test_equal_lengths_keep_the_grid_busy(shape):
     _check(pad.paged_attention_decode(q, k, v, bt, sl), expected, "fp16")
 
 
+def _widest(lens, hkv, heads, groups, d, ps, kv_bytes=2):
+    """Ranges that the longest sequence's first head group spans, in a call of unequal lengths (pa_range.hip's plan)."""
+    page_bytes = ps * d * kv_bytes * 2 * heads
+    extra, least = -(-160 * 1024 // page_bytes), -(-192 * 1024 // page_bytes)
+    pages = [-(-n // ps) for n in lens]
+    assert len({p for p in pages if p}) > 1
+    size = [(p + extra) * (hkv // heads) if p else 0 for p in pages]
+    T = max(-(-sum(size) // groups), least)
+    b = max(range(len(lens)), key=lambda i: pages[i])
+    first = sum(size[:b]) + extra
+    return (first + pages[b] - 1) // T - first // T + 1
+
+
+# One long sequence among empty and one-token ones: its ranges merge in two levels (more than 48), the last of the first
+# level's groups of 16 not full.
+SKEWED = [
+    # (batch, kv heads, group, head_dim, page size, q, kv)
+    (65, 1, 8, 128, 16, "fp16", "fp16"),
+    (33, 8, 4, 128, 16, "bf16", "bf16"),  # four kv heads per workgroup
+    (65, 6, 2, 128, 1, "fp16", "fp16"),  # two
+    (33, 4, 16, 256, 16, "bf16", "bf16"),  # a thread folds several elements
+    (33, 8, 4, 128, 16, "bf16", "e4m3"),
+]
+
+
+def _skewed(case):
+    batch, hkv, group, d, ps, qt, kvt = case
+    lens = [(0, 1, 1)[b % 3] for b in range(batch)]
+    lens[batch // 3] = 32768
+    bt, num_pages = shuffled_table(lens, ps, spare_pages=1, extra_cols=0, seed=d)
+    k, v = make_cache(num_pages, ps, hkv, d, seed=batch)
+    q = torch.randn(batch, hkv * group, d, generator=torch.Generator().manual_seed(ps)).to(DTYPES[qt])
+    return lens, q, k.to(DTYPES[kvt]), v.to(DTYPES[kvt]), bt, torch.tensor(lens, dtype=torch.int32)
+
+
+@pytest.mark.parametrize("case", SKEWED, ids=lambda c: "-".join(map(str, c)))
+def test_skewed_calls_merge_in_two_levels(case):
+    batch, hkv, group, d, ps, _, kvt = case
+    lens = [(0, 1, 1)[b % 3] for b in range(batch)]
+    lens[batch // 3] = 32768
+    es = 1 if kvt == "e4m3" else 2
+    groups, heads, _ = heuristics.range_launch(batch, hkv * group, hkv, d, ps, 32768 // ps, kv_bytes=es)
+    n = _widest(lens, hkv, heads, groups, d, ps, es)
+    assert n > heuristics.TWO_LEVEL_SPLITS and n % 16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", SKEWED, ids=lambda c: "-".join(map(str, c)))
+def test_two_level_fold_against_oracle(case):
+    import paged_attention_decode_amd as pad
+
+    batch, hkv, group, d, ps, qt, kvt = case
+    lens, q, k, v, bt, sl = _skewed(case)
+    expected = decode_fp16_protocol(q.float(), k.float(), v.float(), bt, sl)
+    q, k, v, bt, sl = q.cuda(), k.cuda(), v.cuda(), bt.cuda(), sl.cuda()
+    call = pad.paged_attention_decode_fp8 if kvt == "e4m3" else pad.paged_attention_decode_ex
+    out = call(q, k, v, bt, sl)
+    _check(out, expected, qt)
+    for _ in range(3):  # the group and unit counters are back at zero
+        assert torch.equal(out, call(q, k, v, bt, sl))
+    w = pad.BatchDecodeWrapper()
+    types = dict(q_data_type=DTYPES[qt], kv_data_type=DTYPES[kvt])
+    w.plan_block_table(bt, sl, hkv * group, hkv, d, ps, **types)
+    assert torch.equal(out, w.run(q, (k, v)))
+    indptr, indices, last = pad.paged_kv_indices(bt, sl, ps)
+    csr = pad.paged_attention_decode_csr(q, k, v, indptr, indices, last)
+    _check(csr, expected, qt)
+    w.plan(indptr, indices, last, hkv * group, hkv, d, ps, **types)
+    assert torch.equal(csr, w.run(q, (k, v)))
+    # With counters of its own: zero afterwards.
+    lib = _native.capi()
+    dm = _native.dims_for(q, k, v, bt, sl, out)
+    ws, n = ctypes.c_size_t(), ctypes.c_int64()
+    assert lib.pad_decode_workspace_bytes(ctypes.byref(dm), 0, 0, ctypes.byref(ws)) == 0
+    assert lib.pad_decode_counters_needed(ctypes.byref(dm), 0, 0, ctypes.byref(n)) == 0
+    workspace = torch.empty(ws.value, dtype=torch.uint8, device="cuda")
+    counters = torch.zeros(n.value, dtype=torch.int32, device="cuda")
+    again = torch.empty_like(out)
+    c = _native.PadCall()
+    c.q, c.k_cache, c.v_cache, c.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), again.data_ptr()
+    c.block_table, c.seq_lens = bt.data_ptr(), sl.data_ptr()
+    c.workspace, c.workspace_bytes = workspace.data_ptr(), ws.value
+    c.counters, c.num_counters = counters.data_ptr(), n.value
+    c.scale, c.k_scale, c.v_scale = d ** -0.5, 1.0, 1.0
+    c.kv_format = {("fp16", "fp16"): 0, ("bf16", "bf16"): 3, ("bf16", "e4m3"): 4}[qt, kvt]
+    assert lib.pad_decode_launch_call(ctypes.byref(c), ctypes.byref(dm), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    assert int(counters.abs().sum()) == 0
+
+
+# What the per-unit kernel is tested on, in shapes that take the range kernel: one of each way to address a block.
+FORMS = [("ragged", 40, 4, 4, 128, 16, 2048, "fp16", "fp16"), ("ragged", 40, 4, 4, 128, 12, 2048, "bf16", "bf16"),
+         ("ragged", 40, 4, 4, 128, 4, 2048, "fp16", "e4m3"), ("ragged", 33, 4, 2, 256, 32, 1024, "bf16", "e4m3"),
+         ("ragged", 70, 8, 2, 128, 1, 1024, "bf16", "e5m2"), ("ragged", 70, 6, 2, 96, 16, 2800, "fp16", "fp16")]
+
+
+def _decode(kvt):
+    import paged_attention_decode_amd as pad
+
+    return pad.paged_attention_decode_fp8 if kvt in ("e4m3", "e5m2") else pad.paged_attention_decode_ex
+
+
+def _bits(x):
+    return x.view(torch.uint8) if x.dtype.itemsize == 1 else x
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", FORMS, ids=lambda c: "-".join(map(str, c)))
+def test_strided_views(case):
+    """q, out and both caches as slices of wider tensors, K unlike V, a table and lengths with strides of their own."""
+    kind, batch, hkv, group, d, ps, room, qt, kvt = case
+    lens, q, k, v, bt, sl = _inputs(case)
+    assert heuristics.range_launch(batch, hkv * group, hkv, d, ps, bt.shape[1]) is not None
+    expected = decode_fp16_protocol(q.float(), k.float(), v.float(), bt, sl)
+    dense = _decode(kvt)(q.cuda(), k.cuda(), v.cuda(), bt.cuda(), sl.cuda())
+    qw = torch.zeros(batch, hkv * group, d + 128, dtype=q.dtype, device="cuda")
+    qw[:, :, 64:64 + d] = q.cuda()
+    n = k.shape[0]
+    kw = torch.zeros(n, ps, hkv + 1, d + 8, dtype=k.dtype, device="cuda")
+    _bits(kw)[:, :, :hkv, :d] = _bits(k).cuda()
+    vw = torch.zeros(n, hkv, ps, d + 16, dtype=v.dtype, device="cuda")  # head-major pages
+    _bits(vw)[..., :d] = _bits(v).cuda().transpose(1, 2)
+    btw = torch.full((batch, 2 * bt.shape[1] + 1), -1, dtype=torch.int32, device="cuda")
+    btw[:, :2 * bt.shape[1]:2] = bt.cuda()
+    slw = torch.full((2 * batch,), 1 << 30, dtype=torch.int32, device="cuda")
+    slw[::2] = sl.cuda()
+    out = _decode(kvt)(qw[:, :, 64:64 + d], kw[:, :, :hkv, :d], vw[..., :d].transpose(1, 2),
+                       btw[:, :2 * bt.shape[1]:2], slw[::2])
+    _check(out, expected, qt)
+    assert torch.equal(out, dense)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", FORMS, ids=lambda c: "-".join(map(str, c)))
+def test_nan_in_slots_without_a_token(case):
+    kind, batch, hkv, group, d, ps, room, qt, kvt = case
+    lens, q, k, v, bt, sl = _inputs(case)
+    expected = _decode(kvt)(q.cuda(), k.cuda(), v.cuda(), bt.cuda(), sl.cuda())
+    used = torch.zeros(k.shape[0], ps, dtype=torch.bool)
+    for b, n in enumerate(lens):
+        for p in range(-(-n // ps)):
+            used[int(bt[b, p]), :n - p * ps] = True
+    bad = 0x7F if kvt == "e4m3" else 0x7E if kvt == "e5m2" else float("nan")
+    for x in (k, v):
+        _bits(x)[~used] = bad
+    assert not bool(used.all()) and not bool(torch.isfinite(k.float()).all())
+    assert torch.equal(_decode(kvt)(q.cuda(), k.cuda(), v.cuda(), bt.cuda(), sl.cuda()), expected)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", FORMS[:5], ids=lambda c: "-".join(map(str, c)))
+def test_page_ids_outside_the_cache_read_page_zero(case):
+    kind, batch, hkv, group, d, ps, room, qt, kvt = case
+    lens, q, k, v, bt, sl = _inputs(case)
+    wild, zero = bt.clone(), bt.clone()
+    for i, bad in enumerate((-1, k.shape[0], 2**31 - 1, -2**31)):
+        for b in range(1 + i, batch, 9):
+            col = (7 * b) % bt.shape[1]
+            wild[b, col], zero[b, col] = bad, 0
+    q, k, v, sl = q.cuda(), k.cuda(), v.cuda(), sl.cuda()
+    out = _decode(kvt)(q, k, v, wild.cuda(), sl)
+    assert torch.equal(out, _decode(kvt)(q, k, v, zero.cuda(), sl))
+
+
+@pytest.mark.gpu
+def test_list_of_other_lengths_keeps_the_scratch_consistent():
+    """A range launch's list run with other lengths: rows of the planned items, and the next launches are right."""
+    import paged_attention_decode_amd as pad
+
+    case = FORMS[0]
+    kind, batch, hkv, group, d, ps, room, qt, kvt = case
+    lens, q, k, v, _, _ = _inputs(case)
+    bt, num_pages = shuffled_table([room] * batch, ps, spare_pages=1, extra_cols=0, seed=2)
+    k, v = make_cache(num_pages, ps, hkv, d, seed=3, dtype=torch.float16)
+    other = lens[::-1]
+    sla, slb = (torch.tensor(x, dtype=torch.int32).cuda() for x in (lens, other))
+    qc, kc, vc, btc = q.cuda(), k.cuda(), v.cuda(), bt.cuda()
+    w = pad.BatchDecodeWrapper()
+    w.plan_block_table(btc, sla, hkv * group, hkv, d, ps)
+    stale = pad.ops.ext().forward_worklist(qc, kc, vc, btc, slb, w._plan[2], d ** -0.5, 0)
+    planned = w.run(qc, (kc, vc))
+    assert torch.equal(stale, planned)  # every length comes from the list
+    _check(planned, decode_fp16_protocol(q.float(), k.float(), v.float(), bt, torch.tensor(lens)), qt)
+    out = pad.paged_attention_decode(qc, kc, vc, btc, slb)
+    _check(out, decode_fp16_protocol(q.float(), k.float(), v.float(), bt, torch.tensor(other)), qt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scratch", ["planned", "least"])
+def test_graph_capture_replays(scratch):
+    """Replays equal the eager call's bits; with scratch for the per-unit kernel only, that kernel is captured."""
+    import paged_attention_decode_amd as pad
+
+    # 300 sequences: the per-unit kernel needs no scratch, so a stream without any captures it.
+    batch, hkv, group, d, ps, room = 300, 1, 8, 128, 16, 4096
+    lens, q, k, v, bt, sl = _inputs(("ragged", batch, hkv, group, d, ps, room, "fp16", "fp16"))
+    assert heuristics.plan_units(batch, hkv * group, hkv, d, ps, bt.shape[1]).single_pass
+    assert heuristics.range_launch(batch, hkv * group, hkv, d, ps, bt.shape[1]) is not None
+    expected = decode_fp16_protocol(q.float(), k.float(), v.float(), bt, sl)
+    dev = [k.cuda(), v.cuda(), bt.cuda(), sl.cuda()]
+    qs = [q.cuda(), q.flip(0).contiguous().cuda()]
+    q_static = qs[0].clone()
+    eager = [pad.paged_attention_decode(x, *dev) for x in qs]
+    per_unit = [pad.paged_attention_decode_ex(x, *dev, num_splits=1) for x in qs]
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    if scratch == "planned":
+        with torch.cuda.stream(s):
+            pad.paged_attention_decode(q_static, *dev)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        out = pad.paged_attention_decode(q_static, *dev)
+    for _ in range(3):
+        for i, x in enumerate(qs):
+            q_static.copy_(x)
+            graph.replay()
+            torch.cuda.synchronize()
+            # (the runtime hands out streams again: one of an earlier test may hold more than the least)
+            assert torch.equal(out, eager[i]) or (scratch == "least" and torch.equal(out, per_unit[i]))
+            pad.paged_attention_decode(x, *dev)
+            torch.cuda.synchronize()
+            if i == 0:
+                _check(out, expected, "fp16")
+
+
 def test_plans_describe_one_kernel():
     """Splits, pages and waves of a plan are the per-unit kernel's; its scratch covers the range kernel too."""
     lib = _native.capi()
