@@ -1613,22 +1613,30 @@ constexpr int64_t kRangeMinBytes = 192 * 1024;
 // 30.8 / 26.1 / 24.8 / 22.5 / 23.1 us; 48 x [1, 4096] at page size 1, four
 // layers: 343 / 323 / 314 / 302 / 298 us.
 constexpr int64_t kRangeUnitBytes = 160 * 1024;
-// Fewest K/V bytes of a full table row in one head group.  A workgroup takes
+// Fewest K/V bytes of a full table row in one head group, as 16-bit caches
+// hold them (fp8 rows turn at the same token counts: 200 x [1, n] of 32/8
+// heads, n = 384 / 512 / 640, 0.83 / 1.26 / 1.32 times the per-unit kernel's
+// speed with fp8 and 0.95 / 1.14 / 1.12 with 16-bit caches).  A workgroup takes
 // short units one after the other, several microseconds each, where the
-// per-unit grid runs two or three side by side on a CU: with rows of 0.25 /
-// 0.5 / 0.6 MB the range kernel takes 27.1 / 41.8 / 39.4 us against 18.6 /
-// 36.8 / 34.4 us (200 x [16, 128] of 64/8 heads, 400 x 1000 of 16/1, 256 x [1,
-// 300] of 32/8), from 2 MB on it gains (100 x [1, 1000] of 32/8 45.0 against
-// 49.4 us, 128 x 1024 of 64/8 84.5 against 87.1 us).  The table's width is
-// what the host knows: short sequences in a wide table (the same 200 and 256
-// sequences, rows of 1024 and 4096 tokens) still gain, 27.2 against 35.1 and
-// 39.4 against 57.5 us, as the per-unit grid is then oversubscribed in vain.
+// per-unit grid runs two or three side by side on a CU.  Speed against it at
+// rows of 0.5 / 0.75 / 1 / 1.5 / 2 MB: 200 x [1, n] of 32/8 0.85 / 0.95 / 1.14
+// / 1.16 / 1.15, 128 of 64/8 - / 0.78 / 1.04 / 1.05 / 1.09, 400 of 16/1 at
+// head_dim 256 0.78 / 0.90 / 0.95 / 1.08 / 1.06 (128 of it 0.88-1.03 up to 3).
+// The table's width is what the host knows of a dense call.  Short sequences
+// in a wide table gain where they are many (200 x [1, 300] of 32/8 1.3, the
+// per-unit grid being oversubscribed in vain) and lose where they are few or
+// have one kv head (20 of 32/8 0.8, with fp8 caches 0.6; 100-256 of 8/1 0.8),
+// most above the per-unit planner's batch (300 x [1, 300] of 8/1 10.7 us per
+// unit, 19.6 here; filled to 4096 tokens 76 and 59).
 constexpr int64_t kRangeRowBytes = 3 << 19;
-// Fewest fp16 K/V bytes of all rows: below, the per-unit grid's shorter way to
-// the first load and its smaller merges count for more (us per call, range
-// against per unit: 3 sequences, 38 MB of 32/32 heads, 16.0 against 14.5; 11,
-// 63 MB of 32/8, 21.1 against 19.4; 10, 132 MB of 64/8, 19.8 against 14.6; at
-// 162 MB, 8 of 32/32 with fp8 caches, 16.8 against 38.6).
+// Fewest 16-bit K/V bytes of all rows: below, the per-unit grid's shorter way
+// to the first load and its smaller merges count for more.  Speed against it
+// at 70 / 100 / 134 / 170 / 210 / 270 MB, means of ragged and full tables of 9
+// to 300 sequences: 32/8 heads 0.86 / 0.88 / 0.94 / 0.98 / 1.02 / 1.05, 24/6
+// 0.89 / 0.93 / 0.97 / 1.01 / 1.05 / 1.07, 32/8 at head_dim 64 1.04 / 1.10 /
+// 1.16 / 1.17 / 1.19 / 1.21, 64/8 0.75 / 0.79 / 0.84 / 0.89 / 0.94 / 0.98 (few
+// units among them, which range_shape leaves out; 17 sequences 0.83 / 0.86 /
+// 0.91 / 1.03 / 1.05 / 1.08).
 constexpr int64_t kRangeCallBytes = 1 << 27;
 
 // Takes the calls that the per-unit kernel plans on an oversubscribed grid

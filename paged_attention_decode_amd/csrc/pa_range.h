@@ -7,8 +7,9 @@
 
 namespace pad {
 
-// Largest batch a range launch takes: its planner holds one sequence per lane
-// in up to 8 registers, and its work list two sequences per record.
+// Largest batch a range launch takes: its planner holds a sequence per lane in
+// up to 4 registers (and reads a larger batch twice, in steps), its work list
+// two sequences per record.
 constexpr int kRangeMaxBatch = 512;
 
 // Work list of a range launch: as many int32 per record, and in the header, as

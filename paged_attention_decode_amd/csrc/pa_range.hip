@@ -18,10 +18,11 @@
 //    end and cut into one equal range per workgroup, instead of cutting each
 //    unit into chunks: no chunk is rounded up, so every CU ends at the same
 //    time.  Each unit counts some pages more than it has, at its front: the
-//    time a workgroup takes from one unit to the next.  A workgroup walks its range unit by unit ("segments"); a unit
-//    that lies inside one range is written straight to the output, one that
-//    spans several has one partial per range, folded by the last workgroup
-//    of the unit to arrive (pa_decode.hip's protocol).
+//    time a workgroup takes from one unit to the next.  A workgroup walks its
+//    range unit by unit ("segments"); a unit that lies inside one range is
+//    written straight to the output, one that spans several has one partial
+//    per range, folded by the last workgroup of the unit to arrive
+//    (pa_decode.hip's protocol).
 //
 // See range_wave_loop for the streaming loop.
 
@@ -108,8 +109,8 @@ struct RowLayout {
 
 // 16-token blocks that a wave computes together (see wave_loop_mfma): two, up
 // to head_dim 128.  Two tiles of two blocks of 512-byte rows would not fit the
-// register file, and fp8 caches sum in the order of the 16-bit ones (at unit
-// scales their results are the same bits).
+// register file (fp8 caches go along).  Ranges and waves follow the bytes of
+// the caches, so fp8 results equal 16-bit ones on the same values to rounding.
 template <int D>
 constexpr int tile_blocks() { return D <= 128 ? 2 : 1; }
 
@@ -715,12 +716,11 @@ __device__ __forceinline__ Piece piece_of(const Unit& u, int E, int T, int lo, i
 }
 
 // Work list of a range launch: the header of pa_decode.hip's lists, then one
-// record of 32 int32 per workgroup: {b, head group, first page, page end of
-// the first segment, tokens, ranges of its unit, first of them, pages - 1,
-// valid, CSR row, unit start, T, P, 1 if the workgroup writes zero rows, E, 1
-// unused, raw first page ids of the first segment's first 8 blocks (whole-page
-// blocks), then sequences 2g and 2g + 1 of the batch as {pages, tokens, CSR
-// row, owner of its zero rows or -1}}.
+// record of 32 int32 per workgroup: {b, head group, 2 unused, tokens, 2 unused,
+// pages - 1, valid, CSR row, unit start, T, P, 1 if the workgroup writes zero
+// rows, E, 1 unused, raw first page ids of the first segment's first 8 blocks
+// (whole-page blocks), then sequences 2g and 2g + 1 of the batch as {pages,
+// tokens, CSR row, owner of its zero rows or -1}}.
 constexpr int kRlMagic = 0x574c4150;  // "PALW"
 
 __device__ __forceinline__ const int32_t* list_sequence(const RangeArgs& a, int b) {
@@ -1131,16 +1131,12 @@ __device__ __forceinline__ void write_record(const RangeArgs& a, int32_t* wl) {
   const Unit& u = p.first;
   const int lo = g * p.T, hi = min(lo + p.T, p.P);
   const bool valid = lo < hi;
-  const Piece piece = piece_of(u, p.E, p.T, lo, hi);
+  const int begin = max(lo - u.start - p.E, 0);  // first page of the first segment
   int v = 0;
   switch (lane) {
     case 0: v = u.b; break;
     case 1: v = u.kvh; break;
-    case 2: v = piece.begin; break;
-    case 3: v = piece.end; break;
     case 4: v = u.len; break;
-    case 5: v = piece.n; break;
-    case 6: v = piece.g1; break;
     case 7: v = u.pages - 1; break;
     case 8: v = valid ? 1 : 0; break;
     case 9: v = u.row; break;
@@ -1153,7 +1149,7 @@ __device__ __forceinline__ void write_record(const RangeArgs& a, int32_t* wl) {
   if (!valid) v = 0;
   if (lane == 13) v = zeros != 0 ? 1 : 0;
   if (lane >= 16 && lane < 24 && valid && a.ps % kBlockTokens == 0) {
-    const int col = min(piece.begin + block_page(a, lane - 16), u.pages - 1);
+    const int col = min(begin + block_page(a, lane - 16), u.pages - 1);
     v = a.csr ? a.bt[u.row + col] : a.bt[(int64_t)u.b * a.sbb + (int64_t)col * a.sbp];
   }
   int32_t* r = wl + kRlHeaderInts + (int64_t)kRlRecordInts * g;
