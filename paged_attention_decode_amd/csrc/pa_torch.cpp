@@ -71,11 +71,12 @@ bool stream_capturing(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
-// `least_ws` / `least_counters`: what the launch can do with (the per-unit
+// `least(&ws_bytes, &counters)`: what the launch can do with (the per-unit
 // kernel's scratch); during capture a stream that holds that much is used as
 // it is.
+template <class F>
 StreamScratch& stream_scratch(const torch::Tensor& like, hipStream_t stream, size_t ws_bytes,
-                              int64_t num_counters, size_t least_ws, int64_t least_counters) {
+                              int64_t num_counters, F least) {
   static std::mutex mu;
   static std::map<std::pair<int, uintptr_t>, StreamScratch> cache;
   std::lock_guard<std::mutex> lock(mu);
@@ -85,6 +86,9 @@ StreamScratch& stream_scratch(const torch::Tensor& like, hipStream_t stream, siz
   if ((grow_ws || grow_cnt) && stream_capturing(stream)) {
     const size_t have_ws = sc.workspace.defined() ? static_cast<size_t>(sc.workspace.numel()) : 0;
     const int64_t have_counters = sc.counters.defined() ? sc.counters.numel() : 0;
+    size_t least_ws = 0;
+    int64_t least_counters = 0;
+    least(&least_ws, &least_counters);
     TORCH_CHECK(have_ws >= least_ws && have_counters >= least_counters,
                 "pa_decode: this call needs more split scratch than the capturing stream holds, and scratch "
                 "cannot grow during HIP graph capture (a captured graph keeps the addresses it was captured "
@@ -121,11 +125,10 @@ LaunchScratch launch_scratch(const torch::Tensor& q, hipStream_t stream, const p
                              int cus, bool csr, const pad_decode_plan_t& plan) {
   LaunchScratch s;
   if (plan.single_pass) return s;
-  size_t least_ws = 0;
-  int64_t least_counters = 0;
-  const int st = pad_decode_least_scratch(&d, num_splits, cus, csr ? 1 : 0, &least_ws, &least_counters);
-  TORCH_CHECK(st == PAD_OK, "pa_decode: ", pad_status_string(st));
-  StreamScratch& sc = stream_scratch(q, stream, plan.workspace_bytes, plan.counters, least_ws, least_counters);
+  StreamScratch& sc = stream_scratch(q, stream, plan.workspace_bytes, plan.counters, [&](size_t* ws, int64_t* n) {
+    const int st = pad_decode_least_scratch(&d, num_splits, cus, csr ? 1 : 0, ws, n);
+    TORCH_CHECK(st == PAD_OK, "pa_decode: ", pad_status_string(st));
+  });
   if (sc.workspace.defined() && sc.counters.defined()) {
     s.workspace = sc.workspace.data_ptr();
     s.workspace_bytes = std::min(plan.workspace_bytes, static_cast<size_t>(sc.workspace.numel()));
